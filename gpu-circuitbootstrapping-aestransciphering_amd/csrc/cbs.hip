@@ -6,13 +6,10 @@
 // signed 32-bit limb), rounded and recombined mod 2^64, which is exact, or (the
 // one-product PBS form) one FP64 product of the polynomial scaled to the torus,
 // rounded once.  With a torus-32 polynomial it is one FP64 product, exact.
-#include "fft1024.hpp"
+#include "cbs_device.hpp"
 #include "kernels.hpp"
 
 namespace tfhe {
-
-constexpr int CB_N = 2048, CB_M = 1024;
-constexpr int PBS_LOGB = 9, PBS_L = 4, PBS_ROWS = 8, PBS_IGN = 28;  // PBS gadget (see pbs_digit)
 
 // ---------------------------------------------------------------------------
 // shared helpers
@@ -143,8 +140,6 @@ __global__ __launch_bounds__(256) void k_to_fourier2048_t64(const uint64_t* __re
 // exactly).  LIMBS = 1: the one-product form of the PBS (y scaled to the torus,
 // one FP64 product, rounded once with torus64_from_double); its difference from
 // the exact product is the per-product rounding error of that form.
-__device__ __forceinline__ uint64_t torus64_from_double(double y);
-
 template <int LIMBS>
 __global__ __launch_bounds__(256) void k_polymul2048(const int32_t* __restrict__ x, const uint64_t* __restrict__ y,
                                                     uint32_t batch, FFT1024Tables Tg, uint64_t* __restrict__ out) {
@@ -361,570 +356,6 @@ __global__ __launch_bounds__(256) void k_gen_pfks32(uint64_t seed, uint32_t nrow
             ob[c] = b;
         }
     }
-}
-
-// ===========================================================================
-// Multi-value programmable bootstrap (the circuit bootstrap's blind rotation):
-// one 4-wave workgroup per ciphertext, accumulator in registers in the
-// FFT1024 coefficient ownership.  Input LWE_s (torus-32) of b * 2^31.
-// Steps (reference ManyLUT path, cirbts-batch.cu:3293-4006, restated for the
-// torus-64 CGGI accumulator): b += 2^30; a~_i = special_ms(a_i, bw = 1);
-// test vector with b~ folded in; n CMux steps acc += (X^m - 1)(dec(acc) (*) BSK_i),
-// m = -a~_i mod 2N (or n/2 steps over key-bit pairs, MB = 2); extract
-// coefficients 0 and 1 and add mu_j = 2^(47 + 8j).
-// Output [batch][2][N+1] u64: LWE_K2 of b * 2^(48 + 8j).
-// ===========================================================================
-// PBS gadget: PBS_L = 4 levels of 2^LOGB (LOGB = 9 for every PFKS form, 10 for the
-// HomTrace + SchemeSwitch form), the low 64 - 4 LOGB bits dropped with rounding
-
-// signed digits by the offset method on 64 bits: off = 2^(IGN-1) + sum_j (B/2) 2^(IGN + j logB)
-template <int LOGB, int L>
-__device__ __forceinline__ uint64_t digit_offset64() {
-    constexpr int IGN = 64 - L * LOGB;
-    uint64_t off = 1ull << (IGN - 1);
-#pragma unroll
-    for (int j = 0; j < L; ++j) off += (1ull << (LOGB - 1)) << (IGN + j * LOGB);
-    return off;
-}
-template <int LOGB, int L>
-__device__ __forceinline__ double digit64(uint64_t tp, int j) {
-    constexpr int IGN = 64 - L * LOGB;
-    return (double)((int32_t)((tp >> (IGN + j * LOGB)) & ((1u << LOGB) - 1)) - (1 << (LOGB - 1)));
-}
-
-template <int LOGB = PBS_LOGB>
-__device__ __forceinline__ uint64_t pbs_digit_offset() {
-    return digit_offset64<LOGB, PBS_L>();
-}
-
-template <int LOGB = PBS_LOGB>
-__device__ __forceinline__ double pbs_digit(uint64_t tp, int j) {
-    return digit64<LOGB, PBS_L>(tp, j);
-}
-
-// round(v * 2N / (2^32 2^bw)) * 2^bw mod 2N with N = 2048, bw = 1
-__device__ __forceinline__ uint32_t special_ms_2048(uint32_t v) {
-    return (uint32_t)((((uint64_t)v + (1ull << 20)) >> 21) << 1) & 4095u;
-}
-// the same for any bw in [0, 11] (the reference's gpu_SpecilMS, cirbts-utils.cu:52-61)
-__device__ __forceinline__ uint32_t special_ms_2048_bw(uint32_t v, uint32_t bw) {
-    return (uint32_t)((((uint64_t)v + (1ull << (19 + bw))) >> (20 + bw)) << bw) & 4095u;
-}
-
-// round(y * 2^64) mod 2^64 for a torus value held as a double.  f = y - rint(y)
-// in [-1/2, 1/2] is exact; its top 32 bits are rint(f 2^32), taken with the
-// 1.5 * 2^52 rounding constant, and the exact residual r = f 2^32 - rint(f 2^32)
-// gives the low 32 bits the same way (borrowing one from the top half when
-// rint(r 2^32) < 0, i.e. l < MAGIC).
-__device__ __forceinline__ uint64_t torus64_from_double(double y) {
-    constexpr double MAGIC = 6755399441055744.0, TWO32 = 4294967296.0;
-    const double f = y - rint(y);
-    const double h = fma(f, TWO32, MAGIC);
-    const double r = fma(f, TWO32, -(h - MAGIC));
-    const double l = fma(r, TWO32, MAGIC);
-    const uint32_t hi = (uint32_t)__double_as_longlong(h) - (l < MAGIC ? 1u : 0u);
-    return ((uint64_t)hi << 32) | (uint32_t)__double_as_longlong(l);
-}
-
-// LIMBS = 2: BSK2 Fourier rows hold the two signed 32-bit limbs of each torus-64
-// coefficient and every product is rounded exactly; the monic update rotates the
-// rounded product across the four waves through LDS.  LIMBS = 1: one Fourier row
-// of the coefficients scaled to the torus (k_to_fourier2048_t64); the monic factor
-// is applied pointwise before the inverse transform and the product is rounded
-// once, to about 2^-36 of the torus per step.
-// MB = 2 (one limb only): two key bits per step.  With m1, m2 the rotations of the
-// pair, acc += sum_p (X^(e_p) - 1) (dec(acc) (*) RGSW(ind_p)) over the patterns
-// (1,0), (0,1), (1,1) with e_p = m1, m2, m1 + m2: exactly one indicator is 1 (or
-// none), so this equals the two single-bit steps.  One decomposition and two
-// inverse transforms serve both bits; the factor of pattern p is applied to the
-// digit transforms before they meet that pattern's key row.  The pattern keys are
-// the step's largest load stream (24 complex values per lane and digit row), and the
-// step waits on it unless many loads are in flight: WIDE = false keeps two waves per
-// SIMD and issues each pattern's 8 values as one batch, the next pattern's before the
-// current pattern's MACs; WIDE = true (launches of at most one workgroup per CU)
-// issues all 24 at once with one wave per SIMD.
-template <bool BF, int LIMBS, int MB = 1, bool WIDE = false, bool LUT = false, int LOGB = PBS_LOGB>
-__global__ __launch_bounds__(256, (MB == 2 && !WIDE) ? 2 : 1) void k_pbs2_manylut(const uint32_t* __restrict__ lwe, uint32_t batch, int n,
-                                                     const cplx* __restrict__ bskf, FFT1024Tables Tg,
-                                                     uint64_t* __restrict__ out, PbsLut io) {
-    __shared__ cplx tl[768];
-    __shared__ cplx lds_all[4][F256_LDS_CPLX];
-    __shared__ cplx xbuf[2][1024];
-    __shared__ uint16_t at[1024];
-    const FFT1024Tables T = stage_tables(Tg, tl);
-    const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    cplx trw[4];
-    load_trw(Tg, w, lane, trw);
-    static_assert(MB == 1 || LIMBS == 1, "two key bits per step only in the one-product form");
-    static_assert(!WIDE || MB == 2, "the wide key batch is a form of the two-bit step");
-    constexpr bool RT = LIMBS == 1 && MB == 1;  // registers to spare for the p2 / p3 twiddles
-    const Tw256Regs tw = RT ? load_tw256(Tg, lane) : Tw256Regs{};
-    cplx* lds = lds_all[w];
-    uint64_t* x64 = reinterpret_cast<uint64_t*>(&xbuf[0][0]);  // [2][2048] u64 scratch for the monic exchange
-    const uint64_t OFF = pbs_digit_offset<LOGB>();
-    static_assert(LOGB == PBS_LOGB || (LUT && LIMBS == 2 && MB == 1), "the 2^10 gadget: exact LUT-mode form only");
-    constexpr uint32_t N = CB_N, Q2 = 2 * CB_N;
-    const uint64_t mu0 = 1ull << 47, mu1 = 1ull << 55;
-    uint32_t ek[4];  // evaluation exponents 1 - 4k (mod 2N) of this lane's frequencies
-    const uint32_t kq = (uint32_t)((lane >> 4) + 4 * ((lane >> 2) & 3) + 16 * (lane & 3) + 256 * w);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) ek[s] = (1u - 4u * (kq + 64u * (uint32_t)s)) & (Q2 - 1);
-
-    // MB = 2, two waves per SIMD: the 64 resident workgroups of an XCD each touch one share of
-    // the next step's pattern-key lines after a step's last key load (see k_pbs2_split)
-    constexpr uint32_t KLINES = 3 * PBS_ROWS * 2 * CB_M * sizeof(cplx) / 128;
-    const uint32_t per_xcd = (gridDim.x + 7) / 8 < 64 ? (gridDim.x + 7) / 8 : 64;
-    const uint32_t share = (KLINES + per_xcd - 1) / per_xcd, part = (blockIdx.x >> 3) % per_xcd;
-    uint32_t pf0 = 0, sink = 0;
-    for (uint32_t cidx = blockIdx.x; cidx < batch; cidx += gridDim.x) {
-        const uint32_t* ct = lwe + (size_t)cidx * (n + 1);
-        __syncthreads();
-        uint32_t bt;
-        if constexpr (LUT) {
-            // rotation by X^{+a~_i s_i} (the step multiplies by X^{-at[i]}), so that acc ends
-            // as LUT X^{-phase~}
-            for (int k = threadIdx.x; k < n; k += blockDim.x)
-                at[k] = (uint16_t)((Q2 - special_ms_2048_bw(ct[k], io.bw)) & (Q2 - 1));
-            bt = special_ms_2048_bw(ct[n] + io.b_add, io.bw);
-        } else {
-            for (int k = threadIdx.x; k < n; k += blockDim.x) at[k] = (uint16_t)special_ms_2048(ct[k]);
-            bt = special_ms_2048(ct[n] + (1u << 30));
-        }
-        __syncthreads();
-
-        uint64_t acc[2][8];
-        if constexpr (LUT) {  // acc = (0, LUT X^-bt): coefficient c is LUT[m], m = c + bt mod 2N, negated for m >= N
-#pragma unroll
-            for (int h = 0; h < 8; ++h) {
-                const uint32_t c = (uint32_t)own_coeff(w, lane, h & 3) + (h >= 4 ? CB_M : 0);
-                const uint32_t m = (c + bt) & (Q2 - 1);
-                const uint64_t v = io.lut[m & (N - 1)];
-                acc[0][h] = 0;
-                acc[1][h] = m >= N ? 0 - v : v;
-            }
-        } else {
-#pragma unroll
-            for (int h = 0; h < 8; ++h) {
-                const uint32_t c = (uint32_t)own_coeff(w, lane, h & 3) + (h >= 4 ? CB_M : 0);
-                const uint32_t arg = (bt + Q2 - (c & ~1u)) & (Q2 - 1);
-                uint64_t v = 0 - ((c & 1) ? mu1 : mu0);
-                if (arg >= N) v = 0 - v;
-                acc[0][h] = 0;
-                acc[1][h] = v;
-            }
-        }
-        int buf = 0;
-        for (int i = 0; i < n; i += MB) {
-            const uint32_t mrot = (Q2 - (uint32_t)at[i]) & (Q2 - 1);
-            uint32_t mrot2 = 0;
-            if constexpr (MB == 2) mrot2 = (Q2 - (uint32_t)at[i + 1]) & (Q2 - 1);
-            if ((mrot | mrot2) == 0) continue;
-            const cplx* key = bskf + (size_t)(i / MB) * (MB == 2 ? 3 : 1) * PBS_ROWS * 2 * LIMBS * CB_M;
-            // MB = 2: z1 = w^(m1 (1 - 4k)), z2 = w^(m2 (1 - 4k)); the pattern factors
-            // z1 - 1, z1 z2 - 1 and z2 - 1 (patterns (1,0), (1,1), (0,1)), formed once per step
-            cplx fp[MB == 2 ? 3 : 1][4];
-            if constexpr (MB == 2) {
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const cplx z1 = T.rot[(mrot * ek[s]) & (Q2 - 1)];
-                    const cplx z2 = T.rot[(mrot2 * ek[s]) & (Q2 - 1)];
-                    const cplx z12 = cmul(z1, z2);
-                    fp[0][s] = {z1.re - 1.0, z1.im};
-                    fp[1][s] = {z12.re - 1.0, z12.im};
-                    fp[2][s] = {z2.re - 1.0, z2.im};
-                }
-            }
-            cplx macc[2][LIMBS][4];
-#pragma unroll
-            for (int o = 0; o < 2; ++o)
-#pragma unroll
-                for (int lb = 0; lb < LIMBS; ++lb)
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) macc[o][lb][s] = {0.0, 0.0};
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                uint64_t tp[8];
-#pragma unroll
-                for (int h = 0; h < 8; ++h) tp[h] = acc[u][h] + OFF;
-#pragma unroll
-                for (int j = 0; j < PBS_L; ++j) {
-                    const int r = 2 * j + u;
-                    cplx x[4];
-#pragma unroll
-                    for (int a = 0; a < 4; ++a) x[a] = {pbs_digit<LOGB>(tp[a], j), pbs_digit<LOGB>(tp[a + 4], j)};
-                    f1024_fwd<BF, RT>(x, lds, xbuf[buf], T, trw, w, lane, tw);
-                    buf ^= 1;
-                    if constexpr (MB == 2) {
-                        cplx y[4];
-                        // key values of pattern q (rows in the order (1,0), (1,1), (0,1)) for
-                        // both outputs, issued as batches, which the compiler would otherwise
-                        // split, waiting on each load in turn.
-                        auto load_keys = [&](cplx(&kv)[2][4], int q) {
-                            const int pt = q == 0 ? 0 : q == 1 ? 2 : 1;
-                            const cplx* kr = key + ((size_t)pt * PBS_ROWS + r) * 2 * CB_M + (w * 4) * 64 + lane;
-#pragma unroll
-                            for (int o = 0; o < 2; ++o)
-#pragma unroll
-                                for (int s = 0; s < 4; ++s) kv[o][s] = kr[o * CB_M + s * 64];
-                        };
-                        // WIDE (one wave per SIMD, registers to spare): a scheduling fence keeps a
-                        // batch's loads together and leaves their waits at the first use, so later
-                        // batches are in flight meanwhile.  Two waves per SIMD: the empty asm
-                        // statements wait for the batch at once (both batches in flight at 256
-                        // registers would spill, which measured slower: 2176 inputs 50-51 ms
-                        // against 38)
-                        auto close_batch = [](cplx(&kv)[2][4]) {
-                            if constexpr (WIDE) {
-                                __builtin_amdgcn_sched_barrier(0);
-                            } else {
-#pragma unroll
-                                for (int o = 0; o < 2; ++o)
-#pragma unroll
-                                    for (int k = 0; k < 4; ++k)
-                                        asm volatile("" : "+v"(kv[o][k].re), "+v"(kv[o][k].im));
-                            }
-                        };
-                        auto mac_pattern = [&](const cplx(&kv)[2][4], int q) {
-#pragma unroll
-                            for (int s = 0; s < 4; ++s) y[s] = cmul(x[s], fp[q][s]);
-#pragma unroll
-                            for (int o = 0; o < 2; ++o)
-#pragma unroll
-                                for (int s = 0; s < 4; ++s) cmac(macc[o][0][s], y[s], kv[o][s]);
-                        };
-                        if constexpr (WIDE) {  // all 24 values as one batch
-                            cplx kv[3][2][4];
-#pragma unroll
-                            for (int q = 0; q < 3; ++q) load_keys(kv[q], q);
-#pragma unroll
-                            for (int q = 0; q < 3; ++q) close_batch(kv[q]);
-#pragma unroll
-                            for (int q = 0; q < 3; ++q) mac_pattern(kv[q], q);
-                        } else {  // 8 per batch, pattern q + 1 loaded before pattern q's MACs
-                            cplx ka[2][4], kb[2][4];
-                            load_keys(ka, 0);
-                            close_batch(ka);
-                            load_keys(kb, 1);
-                            close_batch(kb);
-                            mac_pattern(ka, 0);
-                            load_keys(ka, 2);
-                            close_batch(ka);
-                            mac_pattern(kb, 1);
-                            mac_pattern(ka, 2);
-                        }
-                    } else {
-                        const cplx* kr = key + (size_t)r * 2 * LIMBS * CB_M + (w * 4) * 64 + lane;
-#pragma unroll
-                        for (int o = 0; o < 2; ++o)
-#pragma unroll
-                            for (int lb = 0; lb < LIMBS; ++lb)
-#pragma unroll
-                                for (int s = 0; s < 4; ++s)
-                                    cmac(macc[o][lb][s], x[s], kr[(o * LIMBS + lb) * CB_M + s * 64]);
-                    }
-                }
-            }
-            if constexpr (MB == 2 && !WIDE) {
-                sink ^= pf0;
-                const char* nk = reinterpret_cast<const char*>(i + 2 < n ? key + 3 * PBS_ROWS * 2 * CB_M : key);
-                const uint32_t end = (part + 1) * share < KLINES ? (part + 1) * share : KLINES;
-                const uint32_t l0 = part * share + threadIdx.x;
-                pf0 = *reinterpret_cast<const uint32_t*>(nk + (size_t)(l0 < end ? l0 : end - 1) * 128);
-            }
-            if constexpr (LIMBS == 1) {
-                // acc += (X^mrot - 1) t in the Fourier domain: frequency k is the polynomial
-                // at w^(1 - 4k), so t's transform is scaled by w^(mrot (1 - 4k)) - 1 before
-                // the inverse (the product at most doubles; one rounding per coefficient)
-                cplx rf[4];
-                if constexpr (MB == 1) {
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const cplx z = T.rot[(mrot * ek[s]) & (Q2 - 1)];
-                        rf[s] = {z.re - 1.0, z.im};
-                    }
-                }
-#pragma unroll
-                for (int o = 0; o < 2; ++o) {
-                    cplx y0[4];
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) y0[s] = MB == 1 ? cmul(macc[o][0][s], rf[s]) : macc[o][0][s];
-                    f1024_inv<BF, RT>(y0, lds, xbuf[buf], T, trw, w, lane, tw);
-                    buf ^= 1;
-#pragma unroll
-                    for (int a = 0; a < 4; ++a) {
-                        acc[o][a] += torus64_from_double(y0[a].re);
-                        acc[o][a + 4] += torus64_from_double(y0[a].im);
-                    }
-                }
-            } else {
-                uint64_t t[2][8];
-#pragma unroll
-                for (int o = 0; o < 2; ++o) {
-                    cplx y0[4], y1[4];
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) { y0[s] = macc[o][0][s]; y1[s] = macc[o][1][s]; }
-                    f1024_inv<BF>(y0, lds, xbuf[buf], T, trw, w, lane);
-                    buf ^= 1;
-                    f1024_inv<BF>(y1, lds, xbuf[buf], T, trw, w, lane);
-                    buf ^= 1;
-#pragma unroll
-                    for (int a = 0; a < 4; ++a) {
-                        t[o][a] = (uint64_t)round_i64(y0[a].re, 1.0 / CB_M) +
-                                  ((uint64_t)round_i64(y1[a].re, 1.0 / CB_M) << 32);
-                        t[o][a + 4] = (uint64_t)round_i64(y0[a].im, 1.0 / CB_M) +
-                                      ((uint64_t)round_i64(y1[a].im, 1.0 / CB_M) << 32);
-                    }
-                }
-                // acc += X^mrot t - t, rotation across the four waves through LDS
-                __syncthreads();
-#pragma unroll
-                for (int o = 0; o < 2; ++o)
-#pragma unroll
-                    for (int h = 0; h < 8; ++h)
-                        x64[o * CB_N + own_coeff(w, lane, h & 3) + (h >= 4 ? CB_M : 0)] = t[o][h];
-                __syncthreads();
-                const int kshift = (int)(mrot & (N - 1));
-                const bool hi = mrot >= N;
-#pragma unroll
-                for (int o = 0; o < 2; ++o)
-#pragma unroll
-                    for (int h = 0; h < 8; ++h) {
-                        int idx = own_coeff(w, lane, h & 3) + (h >= 4 ? CB_M : 0) - kshift;
-                        const bool wrapped = idx < 0;
-                        idx += wrapped ? (int)N : 0;
-                        uint64_t v = x64[o * CB_N + idx];
-                        if (hi ^ wrapped) v = 0 - v;
-                        acc[o][h] += v - t[o][h];
-                    }
-                __syncthreads();
-            }
-        }
-        if constexpr (LUT) {  // the whole RLWE (mask, body), Gpow_j / 2 added to body coefficient j < 2
-            uint64_t* r = io.rlwe + (size_t)cidx * 2 * N;
-            const uint64_t o0 = io.offsets ? mu0 : 0, o1 = io.offsets ? mu1 : 0;
-#pragma unroll
-            for (int h = 0; h < 8; ++h) {
-                const uint32_t c = (uint32_t)own_coeff(w, lane, h & 3) + (h >= 4 ? CB_M : 0);
-                r[c] = acc[0][h];
-                r[N + c] = acc[1][h] + (c == 0 ? o0 : c == 1 ? o1 : 0);
-            }
-            continue;
-        }
-        // sample extraction of coefficients 0 and 1
-        uint64_t* o0 = out + (size_t)cidx * 2 * (N + 1);
-        uint64_t* o1 = o0 + (N + 1);
-#pragma unroll
-        for (int h = 0; h < 8; ++h) {
-            const uint32_t c = (uint32_t)own_coeff(w, lane, h & 3) + (h >= 4 ? CB_M : 0);
-            const uint64_t v = acc[0][h];
-            o0[(0u - c) & (N - 1)] = (c == 0) ? v : 0 - v;
-            o1[(1u - c) & (N - 1)] = (c <= 1) ? v : 0 - v;
-        }
-        if (lane == 0 && w == 0) o0[N] = acc[1][0] + mu0;
-        if (lane == 0 && w == 1) o1[N] = acc[1][0] + mu1;
-    }
-    if (n < 0) out[threadIdx.x] = sink;  // never (n > 0): keeps the prefetch loads
-}
-
-// Two key bits per step with one ciphertext per 8-wave workgroup (the one-product form):
-// wave group g (waves 4g .. 4g + 3) owns accumulator polynomial g.  Per step each group
-// decomposes its polynomial into the digit rows r = 2j + g, transforms them and sums both
-// outputs' products over its rows; the partial sum of the other group's output goes through
-// LDS, and each group inverse-transforms its own output and updates its polynomial.  A wave
-// runs half the forward transforms and MACs of the 4-wave form per step, and a CU holds two
-// waves per SIMD with one workgroup: the form for launches of at most one workgroup per CU,
-// where the 4-wave forms leave a wave per SIMD.  Each output's sum is the two groups' partial
-// sums added once, where the 4-wave form runs one sum over all eight rows, so the words differ
-// from that form's by FP64 rounding (the phases agree within the one-product form's bound).
-template <bool LUT>
-__global__ __launch_bounds__(512, 1) void k_pbs2_split(const uint32_t* __restrict__ lwe, uint32_t batch, int n,
-                                                      const cplx* __restrict__ bskf, FFT1024Tables Tg,
-                                                      uint64_t* __restrict__ out, PbsLut io) {
-    __shared__ cplx tl[768];
-    __shared__ cplx lds_all[8][F256_LDS_CPLX];
-    __shared__ cplx xbuf[2][2][1024];  // [group][buffer]
-    __shared__ uint16_t at[1024];
-    const FFT1024Tables T = stage_tables(Tg, tl);
-    const int lane = threadIdx.x & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int g = wv >> 2, w = wv & 3;
-    cplx trw[4];
-    load_trw(Tg, w, lane, trw);
-    cplx* lds = lds_all[wv];
-    const uint64_t OFF = pbs_digit_offset<PBS_LOGB>();
-    constexpr uint32_t N = CB_N, Q2 = 2 * CB_N;
-    const uint64_t mu0 = 1ull << 47, mu1 = 1ull << 55;
-    uint32_t ek[4];
-    const uint32_t kq = (uint32_t)((lane >> 4) + 4 * ((lane >> 2) & 3) + 16 * (lane & 3) + 256 * w);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) ek[s] = (1u - 4u * (kq + 64u * (uint32_t)s)) & (Q2 - 1);
-
-    // L2 prefetch of the next step's pattern keys (786 KB): workgroups are dealt to the 8 XCDs
-    // in turn and run the steps nearly in lockstep, so the up to 16 workgroups of one XCD each
-    // touch one share of the step's 128-byte lines (one word per line), issued after the step's
-    // last key loads (loads return in order: earlier, the step's own key waits would include it)
-    // and consumed a step later
-    constexpr uint32_t KLINES = 3 * PBS_ROWS * 2 * CB_M * sizeof(cplx) / 128;
-    const uint32_t per_xcd = (gridDim.x + 7) / 8 < 16 ? (gridDim.x + 7) / 8 : 16;
-    const uint32_t share = (KLINES + per_xcd - 1) / per_xcd, part = (blockIdx.x >> 3) % per_xcd;
-    uint32_t pf0 = 0, pf1 = 0, sink = 0;
-
-    for (uint32_t cidx = blockIdx.x; cidx < batch; cidx += gridDim.x) {
-        const uint32_t* ct = lwe + (size_t)cidx * (n + 1);
-        __syncthreads();
-        uint32_t bt;
-        if constexpr (LUT) {
-            for (int k = threadIdx.x; k < n; k += blockDim.x)
-                at[k] = (uint16_t)((Q2 - special_ms_2048_bw(ct[k], io.bw)) & (Q2 - 1));
-            bt = special_ms_2048_bw(ct[n] + io.b_add, io.bw);
-        } else {
-            for (int k = threadIdx.x; k < n; k += blockDim.x) at[k] = (uint16_t)special_ms_2048(ct[k]);
-            bt = special_ms_2048(ct[n] + (1u << 30));
-        }
-        __syncthreads();
-
-        uint64_t acc[8];  // polynomial g
-#pragma unroll
-        for (int h = 0; h < 8; ++h) {
-            const uint32_t c = (uint32_t)own_coeff(w, lane, h & 3) + (h >= 4 ? CB_M : 0);
-            uint64_t v;
-            if constexpr (LUT) {
-                const uint32_t m = (c + bt) & (Q2 - 1);
-                v = io.lut[m & (N - 1)];
-                if (m >= N) v = 0 - v;
-            } else {
-                const uint32_t arg = (bt + Q2 - (c & ~1u)) & (Q2 - 1);
-                v = 0 - ((c & 1) ? mu1 : mu0);
-                if (arg >= N) v = 0 - v;
-            }
-            acc[h] = g ? v : 0;
-        }
-        int buf = 0;
-        for (int i = 0; i < n; i += 2) {
-            const uint32_t mrot = (Q2 - (uint32_t)at[i]) & (Q2 - 1);
-            const uint32_t mrot2 = (Q2 - (uint32_t)at[i + 1]) & (Q2 - 1);
-            if ((mrot | mrot2) == 0) continue;
-            const cplx* key = bskf + (size_t)(i / 2) * 3 * PBS_ROWS * 2 * CB_M;
-            // z1, z2 per frequency; the pattern factors z1 - 1, z1 z2 - 1, z2 - 1 (patterns
-            // (1,0), (1,1), (0,1)) are formed where they are used, which keeps 16 registers free
-            cplx z1[4], z2[4];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                z1[s] = T.rot[(mrot * ek[s]) & (Q2 - 1)];
-                z2[s] = T.rot[(mrot2 * ek[s]) & (Q2 - 1)];
-            }
-            // sums for this group's output (mown) and the other group's (moth); the key rows
-            // of each are addressed by offset, so no array is indexed by the group
-            cplx mown[4], moth[4];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) mown[s] = moth[s] = {0.0, 0.0};
-            const int own_off = g * CB_M, oth_off = (1 - g) * CB_M;
-            uint64_t tp[8];
-#pragma unroll
-            for (int h = 0; h < 8; ++h) tp[h] = acc[h] + OFF;
-#pragma unroll
-            for (int j = 0; j < PBS_L; ++j) {
-                const int r = 2 * j + g;
-                cplx x[4];
-#pragma unroll
-                for (int a = 0; a < 4; ++a) x[a] = {pbs_digit<PBS_LOGB>(tp[a], j), pbs_digit<PBS_LOGB>(tp[a + 4], j)};
-                f1024_fwd<true>(x, lds, xbuf[g][buf], T, trw, w, lane);
-                buf ^= 1;
-                cplx y[4];
-                auto load_keys = [&](cplx(&kv)[2][4], int q) {
-                    const int pt = q == 0 ? 0 : q == 1 ? 2 : 1;
-                    const cplx* kr = key + ((size_t)pt * PBS_ROWS + r) * 2 * CB_M + (w * 4) * 64 + lane;
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        kv[0][s] = kr[own_off + s * 64];
-                        kv[1][s] = kr[oth_off + s * 64];
-                    }
-                };
-                // a scheduling fence keeps a batch's loads together and leaves their waits at
-                // the first use, so the next batch is in flight meanwhile (1-block AES 18.5 ->
-                // 21.1 blocks/s against waiting for each batch at once)
-                auto close_batch = [](cplx(&)[2][4]) { __builtin_amdgcn_sched_barrier(0); };
-                auto mac_pattern = [&](const cplx(&kv)[2][4], int q) {
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const cplx z = q == 0 ? z1[s] : q == 2 ? z2[s] : cmul(z1[s], z2[s]);
-                        y[s] = cmul(x[s], cplx{z.re - 1.0, z.im});
-                    }
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        cmac(mown[s], y[s], kv[0][s]);
-                        cmac(moth[s], y[s], kv[1][s]);
-                    }
-                };
-                cplx ka[2][4], kb[2][4];
-                load_keys(ka, 0);
-                close_batch(ka);
-                load_keys(kb, 1);
-                close_batch(kb);
-                mac_pattern(ka, 0);
-                load_keys(ka, 2);
-                close_batch(ka);
-                mac_pattern(kb, 1);
-                mac_pattern(ka, 2);
-            }
-            {  // branch-free: the last step re-touches its own key, lines past the share are clamped
-                sink ^= pf0 ^ pf1;  // the previous step's prefetch, long landed
-                const char* nk = reinterpret_cast<const char*>(i + 2 < n ? key + 3 * PBS_ROWS * 2 * CB_M : key);
-                const uint32_t end = (part + 1) * share < KLINES ? (part + 1) * share : KLINES;
-                const uint32_t l0 = part * share + threadIdx.x, l1 = l0 + blockDim.x;
-                pf0 = *reinterpret_cast<const uint32_t*>(nk + (size_t)(l0 < end ? l0 : end - 1) * 128);
-                pf1 = *reinterpret_cast<const uint32_t*>(nk + (size_t)(l1 < end ? l1 : end - 1) * 128);
-            }
-            // the other group's output: this group's partial through LDS (the buffer the
-            // third transform used; the fourth transform's barrier ended its reads)
-            cplx* ex = xbuf[g][buf];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) ex[(w * 4 + s) * 64 + lane] = moth[s];
-            __syncthreads();
-            const cplx* oth = xbuf[1 - g][buf];
-            cplx y0[4];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                y0[s] = cadd(mown[s], oth[(w * 4 + s) * 64 + lane]);
-            }
-            buf ^= 1;
-            // the exchange buffer is read by the other group until that group's inverse
-            // transform reaches its barrier: this transform uses the other buffer
-            f1024_inv<true>(y0, lds, xbuf[g][buf], T, trw, w, lane);
-            buf ^= 1;
-#pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                acc[a] += torus64_from_double(y0[a].re);
-                acc[a + 4] += torus64_from_double(y0[a].im);
-            }
-        }
-        if constexpr (LUT) {
-            uint64_t* r = io.rlwe + (size_t)cidx * 2 * N;
-            const uint64_t o0 = io.offsets ? mu0 : 0, o1 = io.offsets ? mu1 : 0;
-#pragma unroll
-            for (int h = 0; h < 8; ++h) {
-                const uint32_t c = (uint32_t)own_coeff(w, lane, h & 3) + (h >= 4 ? CB_M : 0);
-                r[g * N + c] = acc[h] + (g && c == 0 ? o0 : g && c == 1 ? o1 : 0);
-            }
-            continue;
-        }
-        uint64_t* o0 = out + (size_t)cidx * 2 * (N + 1);
-        uint64_t* o1 = o0 + (N + 1);
-        if (g == 0) {  // sample extraction of coefficients 0 and 1 from the mask polynomial
-#pragma unroll
-            for (int h = 0; h < 8; ++h) {
-                const uint32_t c = (uint32_t)own_coeff(w, lane, h & 3) + (h >= 4 ? CB_M : 0);
-                const uint64_t v = acc[h];
-                o0[(0u - c) & (N - 1)] = (c == 0) ? v : 0 - v;
-                o1[(1u - c) & (N - 1)] = (c <= 1) ? v : 0 - v;
-            }
-        } else {  // bodies: coefficient 0 sits in wave 0, coefficient 1 in wave 1 (lane 0, h = 0)
-            if (lane == 0 && w == 0) o0[N] = acc[0] + mu0;
-            if (lane == 0 && w == 1) o1[N] = acc[0] + mu1;
-        }
-    }
-    if (n < 0) out[threadIdx.x] = sink;  // never (n > 0): keeps the prefetch loads
 }
 
 // ===========================================================================
@@ -1906,67 +1337,6 @@ void launch_aes_linear(const uint32_t* in, const uint32_t* rk, const int16_t* sr
 
 void launch_xor_public(uint32_t* ct, const uint8_t* pub, uint32_t nbits, int n, hipStream_t st) {
     k_xor_public<<<(nbits + 255) / 256, 256, 0, st>>>(ct, pub, nbits, n);
-}
-
-int pbs_model_form(uint32_t batch, int limbs, int mb) {
-    // Two limbs: the branch-free FFT form needs 267 registers (one wave per SIMD),
-    // which pays only up to 256 ciphertexts; beyond, the branchy form keeps two waves
-    // per SIMD.  One limb: the branch-free form fits two waves per SIMD (220
-    // registers) and was the faster one at every size measured.  Two key bits per
-    // step (branch-free FFT): 2 = split over 8 waves, for launches of at most one
-    // workgroup per CU (128 inputs 4.67 ms against 6.20 wide and 6.47 at two waves per
-    // SIMD; 256 inputs 5.08 against 6.22), else 0 = two waves per SIMD (2176 inputs 37.9
-    // against 43.8 split and 54.7 wide); 1 = the wide key batch at one wave per SIMD.
-    if (mb == 2) return batch <= 256 ? 2 : 0;
-    if (limbs == 2) return batch <= 256 ? 1 : 0;
-    return 1;
-}
-
-template <bool LUT>
-static void launch_pbs2_t(const uint32_t* lwe, uint32_t batch, int n, const cplx* bskf, int limbs, int mb,
-                          const FFT1024Tables& T, uint64_t* out, hipStream_t st, int form, const PbsLut& io) {
-    // one workgroup per ciphertext; form: 1 = branch-free cross-wave FFT step,
-    // 0 = branchy (two key bits per step: 1 = wide key batch, 0 = two waves per
-    // SIMD, 2 = split over 8 waves), < 0 = pbs_model_form's choice
-    const unsigned big = grid_for(batch, 2048);
-    if (form < 0) form = pbs_model_form(batch, limbs, mb);
-    if constexpr (LUT) {
-        if (limbs == 2 && io.logB == 10) {  // the HomTrace + SchemeSwitch form's 2^10 x 4 gadget
-            if (form == 1)
-                k_pbs2_manylut<true, 2, 1, false, true, 10><<<batch <= 256 ? batch : big, 256, 0, st>>>(
-                    lwe, batch, n, bskf, T, out, io);
-            else
-                k_pbs2_manylut<false, 2, 1, false, true, 10><<<big, 256, 0, st>>>(lwe, batch, n, bskf, T, out, io);
-            return;
-        }
-    }
-    if (limbs == 2) {
-        if (form == 1)
-            k_pbs2_manylut<true, 2, 1, false, LUT><<<batch <= 256 ? batch : big, 256, 0, st>>>(lwe, batch, n, bskf, T,
-                                                                                               out, io);
-        else
-            k_pbs2_manylut<false, 2, 1, false, LUT><<<big, 256, 0, st>>>(lwe, batch, n, bskf, T, out, io);
-    } else if (mb == 1) {
-        if (form == 0)
-            k_pbs2_manylut<false, 1, 1, false, LUT><<<big, 256, 0, st>>>(lwe, batch, n, bskf, T, out, io);
-        else
-            k_pbs2_manylut<true, 1, 1, false, LUT><<<big, 256, 0, st>>>(lwe, batch, n, bskf, T, out, io);
-    } else if (form == 1) {
-        k_pbs2_manylut<true, 1, 2, true, LUT><<<batch <= 256 ? batch : big, 256, 0, st>>>(lwe, batch, n, bskf, T, out,
-                                                                                          io);
-    } else if (form == 2) {
-        k_pbs2_split<LUT><<<batch <= 256 ? batch : big, 512, 0, st>>>(lwe, batch, n, bskf, T, out, io);
-    } else {
-        k_pbs2_manylut<true, 1, 2, false, LUT><<<big, 256, 0, st>>>(lwe, batch, n, bskf, T, out, io);
-    }
-}
-
-void launch_pbs2(const uint32_t* lwe, uint32_t batch, int n, const cplx* bskf, int limbs, int mb,
-                 const FFT1024Tables& T, uint64_t* out, hipStream_t st, int form, const PbsLut& io) {
-    if (io.lut)
-        launch_pbs2_t<true>(lwe, batch, n, bskf, limbs, mb, T, out, st, form, io);
-    else
-        launch_pbs2_t<false>(lwe, batch, n, bskf, limbs, mb, T, out, st, form, io);
 }
 
 uint32_t pfks_bpad(uint32_t B) { return (B + PF_GROUP - 1) / PF_GROUP * PF_GROUP; }
