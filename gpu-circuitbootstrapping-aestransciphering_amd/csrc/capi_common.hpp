@@ -25,7 +25,7 @@ struct DeviceTables {
     cplx* d_buf = nullptr;
     int init(int N) {
         if (N != 1024) return fail(TFHE_E_PARAM, "FFT tables: only N = 1024 is built");
-        std::vector<cplx> h(2 * 512 + 2 * N);
+        std::vector<cplx> h(1024 + 2 * N + 1024);
         const double PI = 3.14159265358979323846264338327950288;
         for (int k = 0; k < 8; ++k)
             for (int b = 0; b < 64; ++b) {
@@ -42,6 +42,18 @@ struct DeviceTables {
             const double ang = PI * j / N;
             h[1024 + j] = {std::cos(ang), std::sin(ang)};
         }
+        // the two-wave transform: the 256-point step's tables as DeviceTables1024 has them (its
+        // twist exp(4 i pi / 2048) is this one's w^2), then w W512^k at k = 64 f + k0 + 8 e of
+        // lane 8 k0 + e
+        cplx* h2 = h.data() + 1024 + 2 * N;
+        for (int k = 0; k < 4; ++k)
+            for (int l = 0; l < 64; ++l) {
+                auto put = [&](int idx, double ang) { h2[idx + k * 64 + l] = {std::cos(ang), std::sin(ang)}; };
+                put(0, PI * l / 512.0 - 2.0 * PI * (double)((l * k) % 256) / 256.0);
+                put(256, -2.0 * PI * (double)(((l & 15) * k) % 64) / 64.0);
+                put(512, -2.0 * PI * (double)(((l & 3) * k) % 16) / 16.0);
+                put(768, PI / N - 2.0 * PI * (double)(64 * k + (l >> 3) + 8 * (l & 7)) / 512.0);
+            }
         int rc = dmalloc((void**)&d_buf, h.size() * sizeof(cplx));
         if (rc) return rc;
         rc = hipcheck(hipMemcpy(d_buf, h.data(), h.size() * sizeof(cplx), hipMemcpyHostToDevice), "tables");
@@ -49,6 +61,7 @@ struct DeviceTables {
         T.p1t = d_buf;
         T.p2 = d_buf + 512;
         T.rot = d_buf + 1024;
+        T.two = d_buf + 1024 + 2 * N;
         return TFHE_OK;
     }
     void release() {

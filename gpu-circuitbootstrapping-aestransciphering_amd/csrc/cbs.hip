@@ -62,9 +62,9 @@ __global__ __launch_bounds__(256) void k_to_fourier2048(const uint64_t* __restri
             x0[a] = {l0r, l0i};
             x1[a] = {l1r, l1i};
         }
-        f1024_fwd<false>(x0, lds_all[w], xbuf[buf], T, trw, w, lane);
+        f1024_fwd(x0, lds_all[w], xbuf[buf], T, trw, w, lane);
         buf ^= 1;
-        f1024_fwd<false>(x1, lds_all[w], xbuf[buf], T, trw, w, lane);
+        f1024_fwd(x1, lds_all[w], xbuf[buf], T, trw, w, lane);
         buf ^= 1;
         cplx* o = out + q * 2 * CB_M;
 #pragma unroll
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(256) void k_to_fourier2048_32(const uint32_t* __res
             const int c = own_coeff(w, lane, a);
             x[a] = {(double)(int32_t)p[c], (double)(int32_t)p[c + CB_M]};
         }
-        f1024_fwd<false>(x, lds_all[w], xbuf[buf], T, trw, w, lane);
+        f1024_fwd(x, lds_all[w], xbuf[buf], T, trw, w, lane);
         buf ^= 1;
         cplx* o = out + q * CB_M;
 #pragma unroll
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256) void k_to_fourier2048_t64(const uint64_t* __re
             const int c = own_coeff(w, lane, a);
             x[a] = {(double)(int64_t)p[c] * SCALE, (double)(int64_t)p[c + CB_M] * SCALE};
         }
-        f1024_fwd<false>(x, lds_all[w], xbuf[buf], T, trw, w, lane);
+        f1024_fwd(x, lds_all[w], xbuf[buf], T, trw, w, lane);
         buf ^= 1;
         cplx* o = out + q * CB_M;
 #pragma unroll
@@ -171,10 +171,10 @@ __global__ __launch_bounds__(256) void k_polymul2048(const int32_t* __restrict__
                 Y0[a] = {(double)(int64_t)yp[c] * SCALE, (double)(int64_t)yp[c + CB_M] * SCALE};
             }
         }
-        f1024_fwd<false>(X, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
-        f1024_fwd<false>(Y0, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
+        f1024_fwd(X, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
+        f1024_fwd(Y0, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
         if constexpr (LIMBS == 2) {
-            f1024_fwd<false>(Y1, lds_all[w], xbuf[buf], T, trw, w, lane);
+            f1024_fwd(Y1, lds_all[w], xbuf[buf], T, trw, w, lane);
             buf ^= 1;
         }
 #pragma unroll
@@ -182,9 +182,9 @@ __global__ __launch_bounds__(256) void k_polymul2048(const int32_t* __restrict__
             Y0[s] = cmul(Y0[s], X[s]);
             if constexpr (LIMBS == 2) Y1[s] = cmul(Y1[s], X[s]);
         }
-        f1024_inv<false>(Y0, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
+        f1024_inv(Y0, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
         if constexpr (LIMBS == 2) {
-            f1024_inv<false>(Y1, lds_all[w], xbuf[buf], T, trw, w, lane);
+            f1024_inv(Y1, lds_all[w], xbuf[buf], T, trw, w, lane);
             buf ^= 1;
         }
         uint64_t* op = out + (size_t)q * CB_N;
@@ -269,15 +269,15 @@ __global__ __launch_bounds__(256) void k_gen_bsk64(uint64_t seed, uint32_t nrows
             A0[a] = {l0r, l0i};
             A1[a] = {l1r, l1i};
         }
-        f1024_fwd<false>(A0, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
-        f1024_fwd<false>(A1, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
+        f1024_fwd(A0, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
+        f1024_fwd(A1, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
 #pragma unroll
         for (int sl = 0; sl < 4; ++sl) {
             A0[sl] = cmul(A0[sl], kf[sl]);
             A1[sl] = cmul(A1[sl], kf[sl]);
         }
-        f1024_inv<false>(A0, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
-        f1024_inv<false>(A1, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
+        f1024_inv(A0, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
+        f1024_inv(A1, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
         uint64_t* oa = out + (size_t)row * 2 * CB_N;
         uint64_t* ob = oa + CB_N;
 #pragma unroll
@@ -338,10 +338,10 @@ __global__ __launch_bounds__(256) void k_gen_pfks32(uint64_t seed, uint32_t nrow
             av[a + 4] = rand32(seed, DOM_PFKS, id, (uint32_t)(c + CB_M));
             A[a] = {(double)(int32_t)av[a], (double)(int32_t)av[a + 4]};
         }
-        f1024_fwd<false>(A, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
+        f1024_fwd(A, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
 #pragma unroll
         for (int sl = 0; sl < 4; ++sl) A[sl] = cmul(A[sl], kf[sl]);
-        f1024_inv<false>(A, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
+        f1024_inv(A, lds_all[w], xbuf[buf], T, trw, w, lane); buf ^= 1;
         uint32_t* oa = out + (size_t)row * 2 * CB_N;
         uint32_t* ob = oa + CB_N;
 #pragma unroll
@@ -400,7 +400,7 @@ __device__ __forceinline__ void htss_keyswitch(const uint64_t (&x)[8], const cpl
         cplx xd[4];
 #pragma unroll
         for (int a = 0; a < 4; ++a) xd[a] = {digit64<KS_LOGB, KS_L>(tp[a], d), digit64<KS_LOGB, KS_L>(tp[a + 4], d)};
-        f1024_fwd<false>(xd, lds, xbuf[buf], T, trw, w, lane);
+        f1024_fwd(xd, lds, xbuf[buf], T, trw, w, lane);
         buf ^= 1;
         const cplx* kr = key + (size_t)d * 2 * 2 * CB_M + (w * 4) * 64 + lane;
 #pragma unroll
@@ -415,9 +415,9 @@ __device__ __forceinline__ void htss_keyswitch(const uint64_t (&x)[8], const cpl
         cplx y0[4], y1[4];
 #pragma unroll
         for (int s = 0; s < 4; ++s) { y0[s] = macc[o][0][s]; y1[s] = macc[o][1][s]; }
-        f1024_inv<false>(y0, lds, xbuf[buf], T, trw, w, lane);
+        f1024_inv(y0, lds, xbuf[buf], T, trw, w, lane);
         buf ^= 1;
-        f1024_inv<false>(y1, lds, xbuf[buf], T, trw, w, lane);
+        f1024_inv(y1, lds, xbuf[buf], T, trw, w, lane);
         buf ^= 1;
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
@@ -1210,7 +1210,7 @@ __global__ __launch_bounds__(256) void k_lut_vertical(const cplx* __restrict__ r
                     for (int a = 0; a < 4; ++a)
                         x[a] = {(double)((int32_t)((tp[u][a] >> sh2) & 255u) - 128),
                                 (double)((int32_t)((tp[u][a + 4] >> sh2) & 255u) - 128)};
-                    f1024_fwd<false>(x, lds, xbuf[buf], T, trw, w, lane);
+                    f1024_fwd(x, lds, xbuf[buf], T, trw, w, lane);
                     buf ^= 1;
                     const cplx* kr = key + (size_t)r * 2 * CB_M + (w * 4) * 64 + lane;
 #pragma unroll
@@ -1220,7 +1220,7 @@ __global__ __launch_bounds__(256) void k_lut_vertical(const cplx* __restrict__ r
                 }
 #pragma unroll
             for (int o = 0; o < 2; ++o) {
-                f1024_inv<false>(macc[o], lds, xbuf[buf], T, trw, w, lane);
+                f1024_inv(macc[o], lds, xbuf[buf], T, trw, w, lane);
                 buf ^= 1;
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {

@@ -190,6 +190,7 @@ struct FFTTables {
     const cplx* p1t;  // [8][64]
     const cplx* p2;   // [8][64]
     const cplx* rot;  // [2N] w^j, w = exp(i pi / N): X[k] of the transform is p(w^(1 - 4k))
+    const cplx* two;  // two-wave transform: p1t, p2, p3 [4][64] of fft1024.hpp, cross twiddles [4 f][64]
 };
 
 // w^(64a) = exp(i pi a / 16), a = 0..7
@@ -213,6 +214,37 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// the lane index as a value of its own: keeps addresses that are formed once per ciphertext
+// from being hoisted over the step loop, where they would hold registers
+__device__ __forceinline__ int fresh_lane(int lane) {
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+
+// a value equal over the wave, in scalar registers
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+// the same value as one of its own, so that what is formed from it is formed where it is used
+__device__ __forceinline__ uint32_t fresh_uniform(uint32_t v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
+// key value at byte offset `at` of a base that is uniform over the wave; the empty asm keeps
+// the base in scalar registers, instead of a vector addition per load
+__device__ __forceinline__ cplx key_at(const cplx* base, uint32_t at) {
+    typedef double v2d __attribute__((ext_vector_type(2)));
+    auto b = (__attribute__((address_space(1))) const char*)base;
+    asm("" : "+s"(b));
+    const v2d v = *(__attribute__((address_space(1))) const v2d*)(b + at);
+    return {v.x, v.y};
+}
+// LDS-only workgroup barrier: global loads in flight stay in flight across it
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // forward: x = folded coefficient pairs (untwisted), out in frequency distribution

@@ -83,40 +83,46 @@ __device__ __forceinline__ void row_transpose4(C (&x)[4]) {
 __device__ __forceinline__ int f256_a2(int k0, int e, int d) { return k0 * 80 + e * 20 + d; }
 __device__ __forceinline__ int f256_a3(int k0, int e, int p, int h) { return k0 * 80 + e * 20 + p * 5 + h; }
 
-// forward 256-point: x = untwisted folded points (lane b, slot a -> point 64a + b)
-// p2 and p3 twiddles of one lane held in registers (RT = true below): p2[e - 1] =
-// T.p2[64 e + lane], p3[p - 1] = T.p3[64 p + lane]; they are the same for every
-// transform a lane runs, so a kernel with registers to spare loads them once.
+// twiddles of the 256-point step: p1(k), p2(e), p3(p) of one lane, read from the tables ...
 template <class C>
-struct Tw256RegsT {
-    C p2[3], p3[3];
+struct Tw256 {
+    const C *p1t, *p2t, *p3t;  // at this lane
+    __device__ __forceinline__ Tw256(const FFT1024TablesT<C>& T, int lane)
+        : p1t(T.p1t + lane), p2t(T.p2 + lane), p3t(T.p3 + lane) {}
+    __device__ __forceinline__ C p1(int k) const { return p1t[k * 64]; }
+    __device__ __forceinline__ C p2(int e) const { return p2t[e * 64]; }
+    __device__ __forceinline__ C p3(int p) const { return p3t[p * 64]; }
 };
-using Tw256Regs = Tw256RegsT<cplx>;
-
-template <class C>
-__device__ __forceinline__ Tw256RegsT<C> load_tw256(const FFT1024TablesT<C>& T, int lane) {
-    Tw256RegsT<C> r;
+// ... or held in registers: they are the same for every transform a lane runs
+struct Tw256Regs {
+    cplx a[4], b[3], c[3];
+    __device__ __forceinline__ Tw256Regs(const FFT1024Tables& T, int lane) {
 #pragma unroll
-    for (int e = 1; e < 4; ++e) {
-        r.p2[e - 1] = T.p2[e * 64 + lane];
-        r.p3[e - 1] = T.p3[e * 64 + lane];
+        for (int k = 0; k < 4; ++k) a[k] = T.p1t[k * 64 + lane];
+#pragma unroll
+        for (int e = 1; e < 4; ++e) {
+            b[e - 1] = T.p2[e * 64 + lane];
+            c[e - 1] = T.p3[e * 64 + lane];
+        }
     }
-    return r;
-}
+    __device__ __forceinline__ cplx p1(int k) const { return a[k]; }
+    __device__ __forceinline__ cplx p2(int e) const { return b[e - 1]; }
+    __device__ __forceinline__ cplx p3(int p) const { return c[p - 1]; }
+};
 
-template <bool RT, class C>
-__device__ __forceinline__ void fft256_fwd_t(C (&x)[4], C* lds, const FFT1024TablesT<C>& T, const Tw256RegsT<C>& tw,
-                                             int lane) {
+// forward 256-point: x = untwisted folded points (lane b, slot a -> point 64a + b)
+template <class C, class Tw>
+__device__ __forceinline__ void fft256_fwd(C (&x)[4], C* lds, const Tw& T, int lane) {
 #pragma unroll
     for (int a = 1; a < 4; ++a) x[a] = cmul(x[a], twist4_const<C>(a));
     dft4<false>(x);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) x[k] = cmul(x[k], T.p1t[k * 64 + lane]);
+    for (int k = 0; k < 4; ++k) x[k] = cmul(x[k], T.p1(k));
     row_transpose4(x);
     const int k0 = lane >> 4, d = lane & 15;
     dft4<false>(x);
 #pragma unroll
-    for (int e = 1; e < 4; ++e) x[e] = cmul(x[e], RT ? tw.p2[e - 1] : T.p2[e * 64 + lane]);
+    for (int e = 1; e < 4; ++e) x[e] = cmul(x[e], T.p2(e));
 #pragma unroll
     for (int e = 0; e < 4; ++e) lds[f256_a2(k0, e, d)] = x[e];
     wave_sync();
@@ -126,7 +132,7 @@ __device__ __forceinline__ void fft256_fwd_t(C (&x)[4], C* lds, const FFT1024Tab
     wave_sync();
     dft4<false>(x);
 #pragma unroll
-    for (int p = 1; p < 4; ++p) x[p] = cmul(x[p], RT ? tw.p3[p - 1] : T.p3[p * 64 + lane]);
+    for (int p = 1; p < 4; ++p) x[p] = cmul(x[p], T.p3(p));
 #pragma unroll
     for (int p = 0; p < 4; ++p) lds[f256_a3(k0, e, p, h)] = x[p];
     wave_sync();
@@ -137,14 +143,9 @@ __device__ __forceinline__ void fft256_fwd_t(C (&x)[4], C* lds, const FFT1024Tab
     dft4<false>(x);
 }
 
-__device__ __forceinline__ void fft256_fwd(cplx (&x)[4], cplx* lds, const FFT1024Tables& T, int lane) {
-    fft256_fwd_t<false>(x, lds, T, Tw256Regs{}, lane);
-}
-
 // inverse 256-point: frequency layout in, 256 x folded points out
-template <bool RT, class C>
-__device__ __forceinline__ void fft256_inv_t(C (&x)[4], C* lds, const FFT1024TablesT<C>& T, const Tw256RegsT<C>& tw,
-                                             int lane) {
+template <class C, class Tw>
+__device__ __forceinline__ void fft256_inv(C (&x)[4], C* lds, const Tw& T, int lane) {
     dft4<true>(x);
     const int k0 = lane >> 4, e = (lane >> 2) & 3, low = lane & 3;
 #pragma unroll
@@ -154,7 +155,7 @@ __device__ __forceinline__ void fft256_inv_t(C (&x)[4], C* lds, const FFT1024Tab
     for (int p = 0; p < 4; ++p) x[p] = lds[f256_a3(k0, e, p, low)];
     wave_sync();
 #pragma unroll
-    for (int p = 1; p < 4; ++p) x[p] = cmulc(x[p], RT ? tw.p3[p - 1] : T.p3[p * 64 + lane]);
+    for (int p = 1; p < 4; ++p) x[p] = cmulc(x[p], T.p3(p));
     dft4<true>(x);
 #pragma unroll
     for (int g = 0; g < 4; ++g) lds[f256_a2(k0, e, 4 * g + low)] = x[g];
@@ -164,53 +165,24 @@ __device__ __forceinline__ void fft256_inv_t(C (&x)[4], C* lds, const FFT1024Tab
     for (int ee = 0; ee < 4; ++ee) x[ee] = lds[f256_a2(k0, ee, d)];
     wave_sync();
 #pragma unroll
-    for (int ee = 1; ee < 4; ++ee) x[ee] = cmulc(x[ee], RT ? tw.p2[ee - 1] : T.p2[ee * 64 + lane]);
+    for (int ee = 1; ee < 4; ++ee) x[ee] = cmulc(x[ee], T.p2(ee));
     dft4<true>(x);
     row_transpose4(x);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) x[k] = cmulc(x[k], T.p1t[k * 64 + lane]);
+    for (int k = 0; k < 4; ++k) x[k] = cmulc(x[k], T.p1(k));
     dft4<true>(x);
 #pragma unroll
     for (int a = 1; a < 4; ++a) x[a] = cmulc(x[a], twist4_const<C>(a));
 }
 
-__device__ __forceinline__ void fft256_inv(cplx (&x)[4], cplx* lds, const FFT1024Tables& T, int lane) {
-    fft256_inv_t<false>(x, lds, T, Tw256Regs{}, lane);
-}
-
-// Output w of the 4-point DFT across the four waves of an FFT1024,
-// X_w = sum_r y_r W^(r w) with W = -i (forward) or +i (inverse), written as
-// X_w = (y0 + e y2) + W^w (y1 + e y3), e = (-1)^w, W^w = c + i t.  The wave index
-// is uniform, so a select on it compiles to scalar branches that cut the FFT into
-// basic blocks; the constants e, c, t in {0, +-1} make it straight-line FMAs
-// with the same rounding points as the add/subtract form (products by 0 and +-1
-// are exact).
-template <bool INV, class C>
-__device__ __forceinline__ C xwave_dft4(C y0, C y1, C y2, C y3, int w) {
-    using S = decltype(C{}.re);
-    const S e = (w & 1) ? S(-1) : S(1);
-    const S c = (w == 0) ? S(1) : (w == 2) ? S(-1) : S(0);
-    const S tf = (w == 1) ? S(-1) : (w == 3) ? S(1) : S(0);  // sin(-pi w / 2)
-    const S t = INV ? -tf : tf;
-    const C A = {sfma(e, y2.re, y0.re), sfma(e, y2.im, y0.im)};
-    const C B = {sfma(e, y3.re, y1.re), sfma(e, y3.im, y1.im)};
-    return {sfma(-t, B.im, sfma(c, B.re, A.re)), sfma(t, B.re, sfma(c, B.im, A.im))};
-}
-
 // Cross-wave step of the FFT1024 (wave w holds frequencies 256 w ..): forward and
-// inverse, with the cross twiddles trw taken from registers.  The cross-wave
-// radix-4 output of wave w is either selected on w (BF = false: uniform branches,
-// which also bound the scheduler's reordering and keep the one-limb / two-limb
-// kernels within 256 registers, i.e. two waves per SIMD) or computed branch-free
-// (BF = true: fewer instructions and a longer straight-line schedule, but more
-// registers; faster where there is one wave per SIMD anyway).  Both round at the
-// same points, so the outputs are identical.  xbuf: 1024 C of LDS shared by the
-// four waves.
-template <bool BF, bool RT = false, class C>
+// inverse, with the cross twiddles trw taken from registers; the radix-4 output of wave w
+// is selected on w (uniform branches).  xbuf: 1024 C of LDS shared by the four waves.  (The
+// bootstraps run fft_rows.hpp, which computes each radix-4 once.)
+template <class C>
 __device__ __forceinline__ void f1024_fwd(C (&x)[4], C* lds, C* xbuf, const FFT1024TablesT<C>& T,
-                                          const C (&trw)[4], int w, int lane,
-                                          const Tw256RegsT<C>& tw = Tw256RegsT<C>{}) {
-    fft256_fwd_t<RT>(x, lds, T, tw, lane);
+                                          const C (&trw)[4], int w, int lane) {
+    fft256_fwd(x, lds, Tw256<C>(T, lane), lane);
 #pragma unroll
     for (int s = 0; s < 4; ++s) xbuf[(w * 4 + s) * 64 + lane] = cmul(x[s], trw[s]);
     __syncthreads();
@@ -218,19 +190,14 @@ __device__ __forceinline__ void f1024_fwd(C (&x)[4], C* lds, C* xbuf, const FFT1
     for (int s = 0; s < 4; ++s) {
         C y0 = xbuf[(0 * 4 + s) * 64 + lane], y1 = xbuf[(1 * 4 + s) * 64 + lane];
         C y2 = xbuf[(2 * 4 + s) * 64 + lane], y3 = xbuf[(3 * 4 + s) * 64 + lane];
-        if constexpr (BF) {
-            x[s] = xwave_dft4<false>(y0, y1, y2, y3, w);
-        } else {
-            C s02 = cadd(y0, y2), d02 = csub(y0, y2), s13 = cadd(y1, y3), d13 = mul_mi<false>(csub(y1, y3));
-            x[s] = (w == 0) ? cadd(s02, s13) : (w == 1) ? cadd(d02, d13) : (w == 2) ? csub(s02, s13) : csub(d02, d13);
-        }
+        C s02 = cadd(y0, y2), d02 = csub(y0, y2), s13 = cadd(y1, y3), d13 = mul_mi<false>(csub(y1, y3));
+        x[s] = (w == 0) ? cadd(s02, s13) : (w == 1) ? cadd(d02, d13) : (w == 2) ? csub(s02, s13) : csub(d02, d13);
     }
 }
 
-template <bool BF, bool RT = false, class C>
+template <class C>
 __device__ __forceinline__ void f1024_inv(C (&x)[4], C* lds, C* xbuf, const FFT1024TablesT<C>& T,
-                                          const C (&trw)[4], int w, int lane,
-                                          const Tw256RegsT<C>& tw = Tw256RegsT<C>{}) {
+                                          const C (&trw)[4], int w, int lane) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) xbuf[(w * 4 + s) * 64 + lane] = x[s];
     __syncthreads();
@@ -238,16 +205,12 @@ __device__ __forceinline__ void f1024_inv(C (&x)[4], C* lds, C* xbuf, const FFT1
     for (int s = 0; s < 4; ++s) {
         C z0 = xbuf[(0 * 4 + s) * 64 + lane], z1 = xbuf[(1 * 4 + s) * 64 + lane];
         C z2 = xbuf[(2 * 4 + s) * 64 + lane], z3 = xbuf[(3 * 4 + s) * 64 + lane];
-        C y;
-        if constexpr (BF) {
-            y = xwave_dft4<true>(z0, z1, z2, z3, w);
-        } else {
-            C s02 = cadd(z0, z2), d02 = csub(z0, z2), s13 = cadd(z1, z3), d13 = mul_mi<true>(csub(z1, z3));
-            y = (w == 0) ? cadd(s02, s13) : (w == 1) ? cadd(d02, d13) : (w == 2) ? csub(s02, s13) : csub(d02, d13);
-        }
+        C s02 = cadd(z0, z2), d02 = csub(z0, z2), s13 = cadd(z1, z3), d13 = mul_mi<true>(csub(z1, z3));
+        const C y =
+            (w == 0) ? cadd(s02, s13) : (w == 1) ? cadd(d02, d13) : (w == 2) ? csub(s02, s13) : csub(d02, d13);
         x[s] = cmulc(y, trw[s]);
     }
-    fft256_inv_t<RT>(x, lds, T, tw, lane);
+    fft256_inv(x, lds, Tw256<C>(T, lane), lane);
 }
 
 template <class C>

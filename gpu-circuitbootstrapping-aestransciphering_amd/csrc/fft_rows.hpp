@@ -42,13 +42,6 @@ __device__ __forceinline__ RowTables stage_row_tables(const FFT1024Tables& Tg, c
     return {tl, tl + 256, tl + 320};
 }
 
-// LDS-only workgroup barrier: global loads in flight stay in flight across it
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // W16^(h p), h, p in 1..3, the doubles of the p3 table
 __device__ __forceinline__ cplx w16_const(int n) {
     constexpr double K[10][2] = {{1.0, 0.0},

@@ -4,6 +4,7 @@
 #include <atomic>
 
 #include "device_common.hpp"
+#include "fft1024.hpp"
 #include "kernels.hpp"
 
 namespace tfhe {
@@ -269,6 +270,172 @@ __global__ __launch_bounds__(256) void k_gate_blind_rotate(
 }
 
 // ===========================================================================
+// Small batches: one ciphertext per 12-wave workgroup.  With a single wavefront per
+// ciphertext a launch of few gates waits on one wave's chain of 8 transforms per step
+// (6.3 ms for one gate, 6.6 for 256; here 1.9 and 2.1).  Here
+// every FFT512 runs on two waves, 4 points per lane (points 2m + r on wave r; the 256-point
+// step of fft1024.hpp, whose twist is this size's w^2, then Z[k] = Y_0 + T Y_1 and Z[k + 256]
+// = Y_0 - T Y_1 with T = w W512^k):
+//   waves 2 row + r: digit row `row`'s half r;
+//   waves 4 + 2 f + o: the products of output o at frequencies k = 64 f + .. and k + 256, the
+//     radix-2 steps before and after them, and the next step's 12 key values per lane, loaded
+//     while waves 0..3 run the inverse transforms (all at once they would hold up the
+//     products: 98 KB per step through one CU's 64 bytes per cycle);
+//   waves 2 o + r: output o's inverse half r, which holds the accumulator coefficients
+//     2m + r, 2m + r + 512 and publishes their words for the digit rows.
+// Three barriers per step.  Every rounding gives the exact integers of the batched form.
+// ===========================================================================
+constexpr int GSPLIT_WAVES = 2 * GATE_ROWS;
+
+template <bool FUNC>
+__global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_split(
+    const uint32_t* __restrict__ ct1, const uint32_t* __restrict__ ct2, uint32_t batch, int n, int doubled,
+    uint32_t q1, const cplx* __restrict__ bskf, FFTTables Tg, uint32_t* __restrict__ lweN, int logf,
+    const uint32_t* __restrict__ tv) {
+    constexpr int N = GATE_N, M = N / 2;
+    __shared__ cplx bufs[GSPLIT_WAVES][F256_LDS_CPLX];  // transposes, then the half transforms Y_r
+    __shared__ cplx prod[2][2][256];                    // [output][half]
+    __shared__ uint4 accw[2][2][2][64];                 // [poly][half][re, im][lane]: words of slots 0..3
+    __shared__ cplx rot[2 * N];                         // w^j: a gather from global memory takes a line per lane
+    __shared__ uint16_t at[1024];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Tw256Regs T({Tg.two, Tg.two + 256, Tg.two + 512, nullptr, nullptr}, lane);
+    constexpr uint32_t q = 2u * N;
+    constexpr uint32_t OFF = digit_offset32<GATE_LOGB, GATE_L>();
+    const int r = w & 1, row = w >> 1, j = row >> 1, u = row & 1;  // forward role
+    const bool inv = w < 4;                                        // inverse role: output w >> 1, half r
+    const int iv = (w >> 1) & 1;
+    const int f = (w - 4) >> 1, o = w & 1;                         // product role (w >= 4)
+    // the key's frequency lane 8 k0 + e holds k = 64 f + k0 + 8 e; the 256-point step leaves
+    // k = k0' + 4 e' + 16 p' + 64 s at slot s of lane 16 k0' + 4 e' + p'
+    const int kk = (lane >> 3) + 8 * (lane & 7);
+    const int pos = f * 64 + 16 * (kk & 3) + 4 * ((kk >> 2) & 3) + (kk >> 4);
+    const uint32_t ek = (1u - 4u * (uint32_t)(kk + 64 * f)) & (q - 1u);
+    const uint32_t kat = (uint32_t)(o * M + f * 64 + lane) * sizeof(cplx);
+    const cplx cross = Tg.two[768 + (f & 3) * 64 + lane];
+    for (int k = threadIdx.x; k < 2 * N; k += blockDim.x) rot[k] = Tg.rot[k];
+    for (uint32_t cidx = blockIdx.x; cidx < batch; cidx += gridDim.x) {
+        const uint32_t* c1 = ct1 + (size_t)cidx * (n + 1);
+        __syncthreads();
+        const int l0 = fresh_lane(lane);
+        uint32_t acc[8];  // inverse role: words 2 (64 a + lane) + r (slot a), + 512 (slot a + 4)
+        if constexpr (FUNC) {
+            const uint32_t cmask = (q >> logf) - 1u, fmask = (1u << logf) - 1u;
+            for (int k = threadIdx.x; k < n; k += blockDim.x) at[k] = (uint16_t)((c1[k] & cmask) << logf);
+            const uint32_t b = c1[n] & cmask;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const uint32_t c = (uint32_t)(2 * (64 * (s & 3) + l0) + r + (s >= 4 ? M : 0));
+                acc[s] = !iv || (c & fmask) ? 0u : tv[(b - (c >> logf)) & cmask];
+            }
+        } else {
+            const uint32_t* c2 = ct2 + (size_t)cidx * (n + 1);
+            for (int k = threadIdx.x; k < n; k += blockDim.x) {
+                uint32_t v = c1[k] + c2[k];
+                if (doubled) v *= 2u;
+                at[k] = (uint16_t)modswitch_2N(v, 11);
+            }
+            uint32_t vb = c1[n] + c2[n];
+            if (doubled) vb *= 2u;
+            const uint32_t bt = modswitch_2N(vb, 11), q2 = (q1 + N) & (q - 1);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const uint32_t c = (uint32_t)(2 * (64 * (s & 3) + l0) + r + (s >= 4 ? M : 0));
+                acc[s] = iv ? gate_tv(q1, q2, bt, c, q) : 0u;
+            }
+        }
+        auto publish = [&]() {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                accw[iv][r][h][lane] = make_uint4(acc[4 * h], acc[4 * h + 1], acc[4 * h + 2], acc[4 * h + 3]);
+        };
+        // the transform of this wave's half digit row
+        auto forward = [&]() {
+            const uint4 re = accw[u][r][0][lane], im = accw[u][r][1][lane];
+            const uint32_t vr[4] = {re.x, re.y, re.z, re.w}, vi[4] = {im.x, im.y, im.z, im.w};
+            const int sh = 32 - GATE_L * GATE_LOGB + j * GATE_LOGB;
+            constexpr uint32_t BM = (1u << GATE_LOGB) - 1;
+            constexpr int HB = 1 << (GATE_LOGB - 1);
+            cplx x[4];
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                x[a] = {(double)((int32_t)(((vr[a] + OFF) >> sh) & BM) - HB),
+                        (double)((int32_t)(((vi[a] + OFF) >> sh) & BM) - HB)};
+            fft256_fwd(x, bufs[w], T, lane);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) bufs[w][s * 64 + lane] = x[s];
+        };
+        // two loops with the same barriers: merged, the key values in flight would be moved
+        // (and waited for) where the roles' paths join
+        if (w >= 4) {
+            cplx kv[GATE_ROWS][2];  // key values of k and k + 256
+            auto load_keys = [&](int i) {
+                const cplx* key = bskf + (size_t)i * GATE_ROWS * 2 * M;
+#pragma unroll
+                for (int t = 0; t < GATE_ROWS; ++t) {
+                    kv[t][0] = key_at(key + t * 2 * M, kat);
+                    kv[t][1] = key_at(key + t * 2 * M + 256, kat);
+                }
+            };
+            load_keys(0);
+            __syncthreads();
+            for (int i = 0; i < n; ++i) {
+                const uint32_t mrot = (q - uniform(at[i])) & (q - 1);
+                forward();
+                lds_barrier();
+                cplx s0 = {0.0, 0.0}, s1 = {0.0, 0.0};
+#pragma unroll
+                for (int t = 0; t < GATE_ROWS; ++t) {
+                    const cplx y0 = bufs[2 * t][pos], y1 = cmul(bufs[2 * t + 1][pos], cross);
+                    cmac(s0, cadd(y0, y1), kv[t][0]);
+                    cmac(s1, csub(y0, y1), kv[t][1]);
+                }
+                // times w^(m (1 - 4k)) - 1 (exactly 0 for m = 0); w^(m (1 - 4(k + 256))) is (-1)^m of it
+                const cplx z = rot[(mrot * ek) & (q - 1u)];
+                const double sg = (mrot & 1) ? -1.0 : 1.0;
+                s0 = cmul(s0, {z.re - 1.0, z.im});
+                s1 = cmul(s1, {fma(sg, z.re, -1.0), sg * z.im});
+                prod[o][0][pos] = cadd(s0, s1);
+                prod[o][1][pos] = cmulc(csub(s0, s1), cross);
+                lds_barrier();
+                load_keys(i + 1 < n ? i + 1 : i);
+                lds_barrier();
+            }
+        } else {
+            publish();
+            __syncthreads();
+            for (int i = 0; i < n; ++i) {
+                forward();
+                lds_barrier();
+                lds_barrier();
+                cplx x[4];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) x[s] = prod[iv][r][s * 64 + lane];
+                fft256_inv(x, bufs[w], T, lane);
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    acc[a] += round_mod32(x[a].re, 1.0 / M);
+                    acc[a + 4] += round_mod32(x[a].im, 1.0 / M);
+                }
+                publish();
+                lds_barrier();
+            }
+        }
+        const int l1 = fresh_lane(lane);
+        uint32_t* out = lweN + (size_t)cidx * (N + 1);
+        if (inv && iv == 0) {
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const int c = 2 * (64 * (s & 3) + l1) + r + (s >= 4 ? M : 0);
+                out[(N - c) & (N - 1)] = c ? 0u - acc[s] : acc[s];
+            }
+        }
+        if (inv && iv && r == 0 && lane == 0) out[N] = FUNC ? acc[0] : acc[0] + (1u << 29) + 1u;
+    }
+}
+
+// ===========================================================================
 // Plain per-step form (the reference's launch structure, rgsw-acc.cu:606-708):
 // per blind-rotation step a decompose+FFT launch (one wavefront per digit row),
 // a MAC+inverse-FFT launch (one wavefront per output polynomial) and a monic
@@ -519,17 +686,28 @@ void launch_to_fourier1024(const uint32_t* coef, size_t npoly, const FFTTables& 
     k_to_fourier1024<<<(unsigned)((npoly + 3) / 4), 256, 0, st>>>(coef, npoly, T, out);
 }
 
+// Largest batch of the 12-wave form: it takes 1.9-2.1 ms per round of one workgroup per CU,
+// the one-wave form 6.5 ms for up to 4 ciphertexts per CU, so up to three rounds.
+static uint32_t gate_split_max() { return 3 * device_cus(); }
+
 void launch_gate_blind_rotate(const uint32_t* ct1, const uint32_t* ct2, uint32_t batch, int n, int doubled,
                               uint32_t q1, const cplx* bskf, const FFTTables& T, uint32_t* lweN,
                               hipStream_t st) {
-    k_gate_blind_rotate<false><<<(batch + 3) / 4, 256, 0, st>>>(ct1, ct2, batch, n, doubled, q1, bskf, T, lweN,
-                                                                  0, nullptr);
+    if (batch <= gate_split_max())
+        k_gate_blind_rotate_split<false><<<batch, 64 * GSPLIT_WAVES, 0, st>>>(ct1, ct2, batch, n, doubled, q1, bskf, T, lweN, 0,
+                                                                nullptr);
+    else
+        k_gate_blind_rotate<false><<<(batch + 3) / 4, 256, 0, st>>>(ct1, ct2, batch, n, doubled, q1, bskf, T, lweN, 0,
+                                                                    nullptr);
 }
 
 void launch_func_blind_rotate(const uint32_t* ct, uint32_t batch, int n, int logf, const uint32_t* tv,
                               const cplx* bskf, const FFTTables& T, uint32_t* lweN, hipStream_t st) {
-    k_gate_blind_rotate<true><<<(batch + 3) / 4, 256, 0, st>>>(ct, nullptr, batch, n, 0, 0u, bskf, T, lweN, logf,
-                                                                 tv);
+    if (batch <= gate_split_max())
+        k_gate_blind_rotate_split<true><<<batch, 64 * GSPLIT_WAVES, 0, st>>>(ct, nullptr, batch, n, 0, 0u, bskf, T, lweN, logf, tv);
+    else
+        k_gate_blind_rotate<true><<<(batch + 3) / 4, 256, 0, st>>>(ct, nullptr, batch, n, 0, 0u, bskf, T, lweN, logf,
+                                                                     tv);
 }
 
 // LWE arithmetic over power-of-two moduli, element-wise on [batch][n+1] (reference

@@ -21,21 +21,6 @@ __device__ __forceinline__ uint32_t special_ms_2048_bw(uint32_t v, uint32_t bw) 
     return (uint32_t)((((uint64_t)v + (1ull << (19 + bw))) >> (20 + bw)) << bw) & 4095u;
 }
 
-// the lane index as a value of its own: keeps addresses that are formed once per ciphertext
-// from being hoisted over the step loop, where they would hold registers
-__device__ __forceinline__ int fresh_lane(int lane) {
-    asm volatile("" : "+v"(lane));
-    return lane;
-}
-
-// a value equal over the wave, in scalar registers
-__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-// the same value as one of its own, so that what is formed from it is formed where it is used
-__device__ __forceinline__ uint32_t fresh_uniform(uint32_t v) {
-    asm volatile("" : "+s"(v));
-    return v;
-}
-
 // c ? a : b by value (a select of the operands' addresses would keep them in memory)
 __device__ __forceinline__ cplx csel(int c, cplx a, cplx b) { return {c ? a.re : b.re, c ? a.im : b.im}; }
 
@@ -44,15 +29,6 @@ __device__ __forceinline__ uint32_t slot_coeff(int w, int lane, int h) {
     return (uint32_t)own_coeff(w, lane, h & 3) + (h >= 4 ? CB_M : 0);
 }
 
-// key value at byte offset `at` of a base that is uniform over the wave; the empty asm keeps
-// the base in scalar registers, instead of a vector addition per load
-__device__ __forceinline__ cplx key_at(const cplx* base, uint32_t at) {
-    typedef double v2d __attribute__((ext_vector_type(2)));
-    auto b = (__attribute__((address_space(1))) const char*)base;
-    asm("" : "+s"(b));
-    const v2d v = *(__attribute__((address_space(1))) const v2d*)(b + at);
-    return {v.x, v.y};
-}
 // acc + a b, or a b alone for the first product of a sum
 __device__ __forceinline__ void cmac_first(bool first, cplx& acc, cplx a, cplx b) {
     if (first) acc = {fma(-a.im, b.im, a.re * b.re), fma(a.im, b.re, a.re * b.im)};

@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256) void k_polymul2048_split32(const int32_t* __re
             dim[a] = (int64_t)yp[c + SP_M];
             acc[2 * a] = acc[2 * a + 1] = 0u;
         }
-        f1024_fwd<false>(X, lds_all[w], xbuf[buf], T, trw, w, lane);
+        f1024_fwd(X, lds_all[w], xbuf[buf], T, trw, w, lane);
         buf ^= 1;
         int off = 0;
 #pragma unroll
@@ -101,11 +101,11 @@ __global__ __launch_bounds__(256) void k_polymul2048_split32(const int32_t* __re
                 const int32_t li = take_limb(dim[a], wk, last);
                 Y[a] = {(float)lr, (float)li};
             }
-            f1024_fwd<false>(Y, lds_all[w], xbuf[buf], T, trw, w, lane);
+            f1024_fwd(Y, lds_all[w], xbuf[buf], T, trw, w, lane);
             buf ^= 1;
 #pragma unroll
             for (int s = 0; s < 4; ++s) Y[s] = cmul(Y[s], X[s]);
-            f1024_inv<false>(Y, lds_all[w], xbuf[buf], T, trw, w, lane);
+            f1024_inv(Y, lds_all[w], xbuf[buf], T, trw, w, lane);
             buf ^= 1;
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
@@ -150,13 +150,13 @@ __global__ __launch_bounds__(256) void k_polymul2048_fp64_32(const int32_t* __re
             X[a] = {(double)xp[c], (double)xp[c + SP_M]};
             Y[a] = {(double)(int32_t)yp[c], (double)(int32_t)yp[c + SP_M]};
         }
-        f1024_fwd<false>(X, lds_all[w], xbuf[buf], T, trw, w, lane);
+        f1024_fwd(X, lds_all[w], xbuf[buf], T, trw, w, lane);
         buf ^= 1;
-        f1024_fwd<false>(Y, lds_all[w], xbuf[buf], T, trw, w, lane);
+        f1024_fwd(Y, lds_all[w], xbuf[buf], T, trw, w, lane);
         buf ^= 1;
 #pragma unroll
         for (int s = 0; s < 4; ++s) Y[s] = cmul(Y[s], X[s]);
-        f1024_inv<false>(Y, lds_all[w], xbuf[buf], T, trw, w, lane);
+        f1024_inv(Y, lds_all[w], xbuf[buf], T, trw, w, lane);
         buf ^= 1;
         uint32_t* op = out + (size_t)q * SP_N;
 #pragma unroll
