@@ -49,11 +49,16 @@ __device__ __forceinline__ void cmac_first(bool first, cplx& acc, cplx a, cplx b
 //     the two single-bit steps.  One decomposition and two inverse transforms serve both
 //     bits; the factor of pattern p is applied to the digit transforms before they meet that
 //     pattern's key row.
+// The factor of frequency k + 512 is that of k times w^(-2048 m): the same table entry for an
+// even rotation m.  The circuit bootstrap's rotations are even (modulus switch with bw = 1), so
+// a lane looks up half its factors (a lookup is a gather of one cache line per lane); with a
+// caller's bitwidth (ANYM) every factor has its own.
 // Key loads come in batches of 8 values per lane (8 KB per wave): MB = 2: one pattern of one
 // row for both outputs; LIMBS = 2: one output of one row; else one row for both outputs.
-template <int LIMBS, int MB>
+template <int LIMBS, int MB, bool ANYM>
 struct PbsStep {
     static_assert(MB == 1 || LIMBS == 1, "two key bits per step only in the one-product form");
+    static constexpr int NQ = ANYM ? 4 : 2, FP = MB == 2 ? 3 : 1;
     static constexpr int BPR = MB == 2 ? 3 : LIMBS;                 // batches per digit row
     static constexpr int BATCHES = PBS_L * BPR;                     // per accumulator polynomial
     static constexpr size_t KEY = (size_t)(MB == 2 ? 3 : 1) * PBS_ROWS * 2 * LIMBS * CB_M;  // per step
@@ -82,14 +87,13 @@ struct PbsStep {
     }
     // batch t's products; x: the digit transform of its row; fp: pattern factors (MB = 2)
     static __device__ __forceinline__ void mac(cplx (&acc)[2][LIMBS][4], const cplx (&x)[4],
-                                               const cplx (&fp)[MB == 2 ? 3 : 1][4], const cplx (&kv)[2][4], int t,
-                                               bool fresh) {
+                                               const cplx (&fp)[FP][NQ], const cplx (&kv)[2][4], int t, bool fresh) {
         const bool first = fresh && t < LIMBS;
         const int b = t % BPR;
         if constexpr (MB == 2) {
             cplx y[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) y[q] = cmul(x[q], fp[b][q]);
+            for (int q = 0; q < 4; ++q) y[q] = cmul(x[q], fp[b][q % NQ]);
 #pragma unroll
             for (int o = 0; o < 2; ++o)
 #pragma unroll
@@ -105,11 +109,11 @@ struct PbsStep {
         }
     }
     // factors of this lane's frequencies (exponents ek) for the step's rotations
-    static __device__ __forceinline__ void factors(cplx (&fp)[MB == 2 ? 3 : 1][4], const cplx* rot, uint32_t m1,
-                                                   uint32_t m2, const uint32_t (&ek)[4]) {
+    static __device__ __forceinline__ void factors(cplx (&fp)[FP][NQ], const cplx* rot, uint32_t m1, uint32_t m2,
+                                                   const uint32_t (&ek)[4]) {
         constexpr uint32_t Q2 = 2 * CB_N;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < NQ; ++q) {
             const cplx z1 = rot[(m1 * ek[q]) & (Q2 - 1)];
             fp[0][q] = {z1.re - 1.0, z1.im};
             if constexpr (MB == 2) {
@@ -125,11 +129,11 @@ struct PbsStep {
 // The rows of one accumulator polynomial: transforms are in the group's regions, key batches
 // 0 and 1 in flight (ka, kb).  A batch is loaded after the MACs of the batch two before it, so
 // two are in flight or in use at a time (64 registers); the scheduling fences keep it so.
-template <int LIMBS, int MB>
-__device__ __forceinline__ void pbs_mac_rows(cplx (&acc)[2][LIMBS][4], const cplx (&fp)[MB == 2 ? 3 : 1][4],
-                                             cplx (&ka)[2][4], cplx (&kb)[2][4], const cplx* key, uint32_t at, int u, bool fresh,
-                                             int first,                                             int second, const cplx* group, int w, int lane, const cplx (&tr)[3]) {
-    using S = PbsStep<LIMBS, MB>;
+template <class S, int LIMBS>
+__device__ __forceinline__ void pbs_mac_rows(cplx (&acc)[2][LIMBS][4], const cplx (&fp)[S::FP][S::NQ],
+                                             cplx (&ka)[2][4], cplx (&kb)[2][4], const cplx* key, uint32_t at, int u,
+                                             bool fresh, int first, int second, const cplx* group, int w, int lane,
+                                             const cplx (&tr)[3]) {
     cplx x[4];
 #pragma unroll
     for (int t = 0; t < S::BATCHES; ++t) {
@@ -272,7 +276,7 @@ template <bool LUT>
 __global__ __launch_bounds__(256, 2) void k_pbs2(const uint32_t* __restrict__ lwe, uint32_t batch, int n,
                                                 const cplx* __restrict__ bskf, FFT1024Tables Tg,
                                                 uint64_t* __restrict__ out, PbsLut io) {
-    using S = PbsStep<1, 1>;
+    using S = PbsStep<1, 1, LUT>;
     __shared__ cplx regions[4][ROWS_CPLX];
     __shared__ cplx tl[ROW_TABLES_CPLX];
     __shared__ uint16_t at[1024];
@@ -303,7 +307,7 @@ __global__ __launch_bounds__(256, 2) void k_pbs2(const uint32_t* __restrict__ lw
             const uint32_t m1 = (Q2 - uniform(at[i])) & (Q2 - 1);
             if (m1 == 0) continue;
             const cplx* step = bskf + (size_t)i * S::KEY;
-            cplx fp[1][4];
+            cplx fp[S::FP][S::NQ];
             cplx macc[2][1][4];
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
@@ -319,14 +323,14 @@ __global__ __launch_bounds__(256, 2) void k_pbs2(const uint32_t* __restrict__ lw
                 S::load(ka, step, kat, u, 0, 0, 1);
                 S::load(kb, step, kat, u, 1, 0, 1);
                 lds_barrier();
-                pbs_mac_rows<1, 1>(macc, fp, ka, kb, step, kat, u, u == 0, 0, 1, &regions[0][0], w, lane, tr);
+                pbs_mac_rows<S>(macc, fp, ka, kb, step, kat, u, u == 0, 0, 1, &regions[0][0], w, lane, tr);
             }
             next.touch(i + 1 < n ? step + S::KEY : step);
             S::factors(fp, Tg.rot, m1, 0, ek);
 #pragma unroll
             for (int o = 0; o < 2; ++o) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) macc[o][0][q] = cmul(macc[o][0][q], fp[0][q]);
+                for (int q = 0; q < 4; ++q) macc[o][0][q] = cmul(macc[o][0][q], fp[0][q % S::NQ]);
                 cross_inv(macc[o][0], tr);
             }
             lds_barrier();  // every wave has read the digit transforms
@@ -362,12 +366,13 @@ __global__ __launch_bounds__(256, 2) void k_pbs2(const uint32_t* __restrict__ lw
 // with hp = wv >> 2, of BOTH ciphertexts, so that one key load feeds two products: the key
 // stream (196 KB per wave and step in the two-bit form when each ciphertext loads its own) is
 // what a step waits on most at this size of launch.
-template <int LIMBS, int MB>
+template <int LIMBS, int MB, bool ANYM>
 struct PbsPair {
-    using S = PbsStep<LIMBS, MB>;
+    using S = PbsStep<LIMBS, MB, ANYM>;
+    static constexpr int NQ = ANYM ? 2 : 1;
     static constexpr int DEPTH = MB == 2 ? 2 : 4;  // key batches in flight
     cplx macc[2][2][LIMBS][2];       // [ciphertext][output][limb][q]
-    cplx fp[2][MB == 2 ? 3 : 1][2];
+    cplx fp[2][S::FP][NQ];
 
     static __device__ __forceinline__ void load(cplx (&kv)[4], const cplx* key, uint32_t at, int u, int t) {
         const int j = t / S::BPR, b = t % S::BPR, r = 2 * j + u;
@@ -394,7 +399,7 @@ struct PbsPair {
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 if constexpr (MB == 2) {
-                    const cplx y = cmul(x[c][q], fp[c][b][q]);
+                    const cplx y = cmul(x[c][q], fp[c][b][q % NQ]);
 #pragma unroll
                     for (int o = 0; o < 2; ++o) cmac_first(first, macc[c][o][0][q], y, kv[2 * o + q]);
                 } else {
@@ -409,7 +414,7 @@ struct PbsPair {
     __device__ __forceinline__ void factors(const cplx* rot, int c, uint32_t m1, uint32_t m2, const uint32_t (&ek)[2]) {
         constexpr uint32_t Q2 = 2 * CB_N;
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
+        for (int q = 0; q < NQ; ++q) {
             const cplx z1 = rot[(m1 * ek[q]) & (Q2 - 1)];
             fp[c][0][q] = {z1.re - 1.0, z1.im};
             if constexpr (MB == 2) {
@@ -426,8 +431,8 @@ template <int LIMBS, int MB, bool LUT, int LOGB = PBS_LOGB>
 __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict__ lwe, uint32_t batch, int n,
                                                      const cplx* __restrict__ bskf, FFT1024Tables Tg,
                                                      uint64_t* __restrict__ out, PbsLut io) {
-    using S = PbsStep<LIMBS, MB>;
-    using P = PbsPair<LIMBS, MB>;
+    using S = PbsStep<LIMBS, MB, LUT>;
+    using P = PbsPair<LIMBS, MB, LUT>;
     __shared__ cplx regions[8][ROWS_CPLX];
     __shared__ cplx tl[ROW_TABLES_CPLX];
     __shared__ uint16_t at[2][1024];
@@ -489,6 +494,10 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict
             if ((m1[0] | m1[1] | m2[0] | m2[1]) == 0) continue;
             const cplx* step = bskf + (size_t)(i / MB) * S::KEY;
             P pr;
+            if constexpr (MB == 2 && !LUT) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c) pr.factors(Tg.rot, c, m1[c], m2[c], ek);
+            }
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 {
@@ -502,7 +511,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict
                 cplx kv[P::DEPTH][4];
 #pragma unroll
                 for (int t = 0; t < P::DEPTH; ++t) P::load(kv[t], step, kat, u, t);
-                if constexpr (MB == 2) {
+                if constexpr (MB == 2 && LUT) {
                     // formed for each polynomial: they would hold 48 registers over the transforms
 #pragma unroll
                     for (int c = 0; c < 2; ++c) pr.factors(Tg.rot, c, fresh_uniform(m1[c]), fresh_uniform(m2[c]), ek);
@@ -539,7 +548,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict
                         for (int lb = 0; lb < LIMBS; ++lb)
 #pragma unroll
                             for (int q = 0; q < 2; ++q)
-                                pr.macc[c][o][lb][q] = cmul(pr.macc[c][o][lb][q], pr.fp[c][0][q]);
+                                pr.macc[c][o][lb][q] = cmul(pr.macc[c][o][lb][q], pr.fp[c][0][q % P::NQ]);
                 }
             }
             // each wave gives the other ciphertext's sums to wave wv ^ 4 and gets its own
@@ -629,7 +638,7 @@ template <int LIMBS, int MB, bool LUT, int LOGB = PBS_LOGB>
 __global__ __launch_bounds__(512, 1) void k_pbs2_split(const uint32_t* __restrict__ lwe, uint32_t batch, int n,
                                                       const cplx* __restrict__ bskf, FFT1024Tables Tg,
                                                       uint64_t* __restrict__ out, PbsLut io) {
-    using S = PbsStep<LIMBS, MB>;
+    using S = PbsStep<LIMBS, MB, LUT>;
     __shared__ cplx regions[8][ROWS_CPLX];
     __shared__ cplx tl[ROW_TABLES_CPLX];
     __shared__ uint16_t at[1024];
@@ -664,7 +673,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_split(const uint32_t* __restric
             if constexpr (MB == 2) m2 = (Q2 - uniform(at[i + 1])) & (Q2 - 1);
             if ((m1 | m2) == 0) continue;
             const cplx* step = bskf + (size_t)(i / MB) * S::KEY;
-            cplx fp[MB == 2 ? 3 : 1][4];
+            cplx fp[S::FP][S::NQ];
             if constexpr (MB == 2) S::factors(fp, Tg.rot, m1, m2, ek);
             cplx macc[2][LIMBS][4];  // this group's output, the other group's
             cplx ka[2][4], kb[2][4];
@@ -676,7 +685,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_split(const uint32_t* __restric
             S::load(ka, step, kat, g, 0, g, 1 - g);
             S::load(kb, step, kat, g, 1, g, 1 - g);
             lds_barrier();
-            pbs_mac_rows<LIMBS, MB>(macc, fp, ka, kb, step, kat, g, true, g, 1 - g, group, w, lane, tr);
+            pbs_mac_rows<S>(macc, fp, ka, kb, step, kat, g, true, g, 1 - g, group, w, lane, tr);
             next.touch(i + MB < n ? step + S::KEY : step);
             lds_barrier();  // every wave has read the digit transforms
 #pragma unroll
@@ -694,7 +703,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_split(const uint32_t* __restric
 #pragma unroll
                 for (int lb = 0; lb < LIMBS; ++lb)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) macc[0][lb][q] = cmul(macc[0][lb][q], fp[0][q]);
+                    for (int q = 0; q < 4; ++q) macc[0][lb][q] = cmul(macc[0][lb][q], fp[0][q % S::NQ]);
             }
             // the exchange of the inverse transform in the regions' second half (the first still
             // holds the partial sums that the other group reads)
