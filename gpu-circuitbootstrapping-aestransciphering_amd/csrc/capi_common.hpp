@@ -11,6 +11,7 @@
 #include "../../include/tfhe_amd.h"
 #include "device_common.hpp"
 #include "fft1024.hpp"
+#include "fft512_pair.hpp"
 
 namespace tfhe {
 
@@ -25,7 +26,7 @@ struct DeviceTables {
     cplx* d_buf = nullptr;
     int init(int N) {
         if (N != 1024) return fail(TFHE_E_PARAM, "FFT tables: only N = 1024 is built");
-        std::vector<cplx> h(1024 + 2 * N + 1024);
+        std::vector<cplx> h(1024 + 2 * N + 1024 + PAIR_TABLE_CPLX);
         const double PI = 3.14159265358979323846264338327950288;
         for (int k = 0; k < 8; ++k)
             for (int b = 0; b < 64; ++b) {
@@ -43,8 +44,7 @@ struct DeviceTables {
             h[1024 + j] = {std::cos(ang), std::sin(ang)};
         }
         // the two-wave transform: the 256-point step's tables as DeviceTables1024 has them (its
-        // twist exp(4 i pi / 2048) is this one's w^2), then w W512^k at k = 64 f + k0 + 8 e of
-        // lane 8 k0 + e
+        // twist exp(4 i pi / 2048) is this one's w^2), then w W512^k, k < 256
         cplx* h2 = h.data() + 1024 + 2 * N;
         for (int k = 0; k < 4; ++k)
             for (int l = 0; l < 64; ++l) {
@@ -52,8 +52,23 @@ struct DeviceTables {
                 put(0, PI * l / 512.0 - 2.0 * PI * (double)((l * k) % 256) / 256.0);
                 put(256, -2.0 * PI * (double)(((l & 15) * k) % 64) / 64.0);
                 put(512, -2.0 * PI * (double)(((l & 3) * k) % 16) / 16.0);
-                put(768, PI / N - 2.0 * PI * (double)(64 * k + (l >> 3) + 8 * (l & 7)) / 512.0);
+                put(768, PI / N - 2.0 * PI * (double)(64 * k + l) / 512.0);
             }
+        // the two-transforms-per-wave form (fft512_pair.hpp): square roots down the tree below
+        // node n = (b1 b2 b3 b4), whose root angle is th
+        cplx* h3 = h2 + 1024;
+        for (int n = 0; n < 16; ++n) {
+            const double th = PI / 32 + PI * (((n >> 3) & 1) / 8.0 + ((n >> 2) & 1) / 4.0 + ((n >> 1) & 1) / 2.0 + (n & 1));
+            auto put = [&](int idx, double ang) { h3[idx] = {std::cos(ang), std::sin(ang)}; };
+            put(n, th / 2);
+            put(16 + n, th / 4);
+            for (int b = 0; b < 2; ++b) put(32 + 16 * b + n, th / 8 + PI * b / 4);
+            for (int b = 0; b < 4; ++b) put(64 + 16 * b + n, th / 16 + PI * ((b >> 1) / 8.0 + (b & 1) / 4.0));
+            for (int p = 0; p < 8; ++p)
+                for (int b8 = 0; b8 < 2; ++b8)
+                    put(128 + 32 * p + n + 16 * b8, th / 32 + PI * ((p >> 2) / 16.0 + ((p >> 1) & 1) / 8.0 + (p & 1) / 4.0) +
+                                                        PI / 2 * b8);
+        }
         int rc = dmalloc((void**)&d_buf, h.size() * sizeof(cplx));
         if (rc) return rc;
         rc = hipcheck(hipMemcpy(d_buf, h.data(), h.size() * sizeof(cplx), hipMemcpyHostToDevice), "tables");
@@ -62,6 +77,7 @@ struct DeviceTables {
         T.p2 = d_buf + 512;
         T.rot = d_buf + 1024;
         T.two = d_buf + 1024 + 2 * N;
+        T.pair = T.two + 1024;
         return TFHE_OK;
     }
     void release() {

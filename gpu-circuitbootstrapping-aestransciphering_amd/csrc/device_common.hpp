@@ -190,7 +190,8 @@ struct FFTTables {
     const cplx* p1t;  // [8][64]
     const cplx* p2;   // [8][64]
     const cplx* rot;  // [2N] w^j, w = exp(i pi / N): X[k] of the transform is p(w^(1 - 4k))
-    const cplx* two;  // two-wave transform: p1t, p2, p3 [4][64] of fft1024.hpp, cross twiddles [4 f][64]
+    const cplx* pair;  // twiddles of fft512_pair.hpp
+    const cplx* two;  // two-wave transform: p1t, p2, p3 [4][64] of fft1024.hpp, cross twiddles [256]
 };
 
 // w^(64a) = exp(i pi a / 16), a = 0..7
@@ -231,8 +232,9 @@ __device__ __forceinline__ uint32_t fresh_uniform(uint32_t v) {
     return v;
 }
 
-// key value at byte offset `at` of a base that is uniform over the wave; the empty asm keeps
-// the base in scalar registers, instead of a vector addition per load
+// key value at byte offset `at` of a base that is uniform over the wave.  The empty asm keeps
+// the base in scalar registers; with the offset from fresh_offset in the same block the load
+// takes both as they are (instead of a 64-bit vector addition per load).
 __device__ __forceinline__ cplx key_at(const cplx* base, uint32_t at) {
     typedef double v2d __attribute__((ext_vector_type(2)));
     auto b = (__attribute__((address_space(1))) const char*)base;
@@ -240,6 +242,13 @@ __device__ __forceinline__ cplx key_at(const cplx* base, uint32_t at) {
     const v2d v = *(__attribute__((address_space(1))) const v2d*)(b + at);
     return {v.x, v.y};
 }
+// a lane's 32-bit offset as a value of the block it is used in (once per batch of loads): one
+// widened outside the loop would hide that it fits 32 bits
+__device__ __forceinline__ uint32_t fresh_offset(uint32_t at) {
+    asm("" : "+v"(at));
+    return at;
+}
+
 // LDS-only workgroup barrier: global loads in flight stay in flight across it
 __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -303,10 +312,19 @@ __device__ __forceinline__ void fft512_inv(cplx (&x)[8], cplx* lds, const FFTTab
     for (int a = 1; a < 8; ++a) x[a] = cmulc(x[a], twist_const(a));
 }
 
+constexpr double ROUND_MAGIC = 6755399441055744.0;  // 1.5 * 2^52
+// ROUND_MAGIC in vector registers, for loops that round many values: as a literal it takes two
+// moves at every use (an FMA reads one scalar operand)
+__device__ __forceinline__ double round_magic() {
+    double m = ROUND_MAGIC;
+    asm volatile("" : "+v"(m));
+    return m;
+}
+
 // round(x * scale) mod 2^32 for |x * scale| < 2^51: adding 1.5 * 2^52 leaves the
 // rounded integer (ties to even, as rint) in the low mantissa bits.
-__device__ __forceinline__ uint32_t round_mod32(double x, double scale) {
-    const double y = fma(x, scale, 6755399441055744.0);
+__device__ __forceinline__ uint32_t round_mod32(double x, double scale, double magic = ROUND_MAGIC) {
+    const double y = fma(x, scale, magic);
     return (uint32_t)__double_as_longlong(y);
 }
 

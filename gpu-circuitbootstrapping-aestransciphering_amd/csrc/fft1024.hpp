@@ -224,18 +224,9 @@ __device__ __forceinline__ int own_coeff(int w, int lane, int a) { return 4 * (6
 
 // round(x * scale) mod 2^64 through two FP64 limbs is done by the callers;
 // exact int64 of a rounded double with |x| < 2^52.
-constexpr double ROUND_MAGIC = 6755399441055744.0;  // 1.5 * 2^52
 __device__ __forceinline__ int64_t round_i64(double x, double scale, double magic = ROUND_MAGIC) {
     const double y = fma(x, scale, magic);
     return __double_as_longlong(y) - 0x4338000000000000ll;
-}
-
-// ROUND_MAGIC in vector registers, for loops that round many values: as a literal it takes two
-// moves at every use (an FMA reads one scalar operand)
-__device__ __forceinline__ double round_magic() {
-    double m = ROUND_MAGIC;
-    asm volatile("" : "+v"(m));
-    return m;
 }
 
 }  // namespace tfhe

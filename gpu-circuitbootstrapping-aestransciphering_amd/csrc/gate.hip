@@ -5,6 +5,7 @@
 
 #include "device_common.hpp"
 #include "fft1024.hpp"
+#include "fft512_pair.hpp"
 #include "kernels.hpp"
 
 namespace tfhe {
@@ -86,8 +87,8 @@ __global__ __launch_bounds__(256) void k_gen_ksk32(uint64_t seed, uint32_t dom, 
 }
 
 // ===========================================================================
-// Fourier conversion of N=1024 torus-32 polynomials into the kernel frequency
-// layout [poly][slot 8][lane 64] (one wavefront per polynomial).
+// Fourier conversion of N=1024 torus-32 polynomials into the key's frequency order
+// (fft512_pair.hpp), [poly][p 8][lane 64] (one wavefront per polynomial).
 // ===========================================================================
 __global__ __launch_bounds__(256) void k_to_fourier1024(const uint32_t* __restrict__ coef, size_t npoly,
                                                        FFTTables T, cplx* __restrict__ out) {
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(256) void k_to_fourier1024(const uint32_t* __restri
     fft512_fwd(x, lds, T, lane);
     cplx* o = out + q * 512;
 #pragma unroll
-    for (int f = 0; f < 8; ++f) o[f * 64 + lane] = x[f];
+    for (int f = 0; f < 8; ++f) o[pair_pos((uint32_t)((lane >> 3) + 8 * (lane & 7) + 64 * f))] = x[f];
 }
 
 // ===========================================================================
@@ -126,11 +127,15 @@ __device__ __forceinline__ uint32_t gate_tv(uint32_t q1, uint32_t q2, uint32_t b
 }
 
 // ===========================================================================
-// Persistent batched gate bootstrap: one wavefront owns one ciphertext for all
-// n blind-rotation steps.  Per step: signed decomposition of the register-
-// resident accumulator, 6 forward FFTs with the Fourier-domain MAC against the
-// streamed BSK row block, 2 inverse FFTs, exact rounding mod 2^32 and the CGGI
-// monic update acc += X^m t - t with m = -a~_i mod 2N (reference
+// Persistent batched gate bootstrap: one wavefront owns one ciphertext for all n
+// blind-rotation steps, half-wave u its accumulator polynomial u.  Bound by FP64 issue (2,388
+// FP64 of 3,080 vector instructions per step, two waves per SIMD: 77% of the issue slots at
+// the clock the chip holds under FMA load).  With one radix-8 transform per wave at a time
+// (two LDS round trips each, eight in a row) 1000 / 2048 / 4096 gates took 6.5 / 11.2 / 21.2 ms;
+// now 6.2 / 10.5 / 19.9.  Per step: the digit rows
+// of both polynomials by pairs (fft512_pair.hpp), the Fourier-domain MAC against the
+// streamed BSK row block, the two inverse transforms as one pair, exact rounding mod 2^32 and
+// the CGGI monic update acc += X^m t - t with m = -a~_i mod 2N (reference
 // rgsw-acc.cu:606-708 fused into one launch).  Ends with sample extraction
 // (coefficient 0) and the + Q/8 + 1 offset; the key switch runs separately.
 // ===========================================================================
@@ -141,132 +146,169 @@ constexpr int GATE_N = 1024, GATE_LOGB = 7, GATE_L = 3, GATE_ROWS = 6;
 // rounding), test vector m[j 2^logf] = tv[(b - j) mod ctmod] for j < ctmod / 2 (tv already scaled
 // to the torus by the host) and zero elsewhere, no offset after extraction.
 template <bool FUNC>
-__global__ __launch_bounds__(256) void k_gate_blind_rotate(
+__global__ __launch_bounds__(256, 2) void k_gate_blind_rotate(
     const uint32_t* __restrict__ ct1, const uint32_t* __restrict__ ct2, uint32_t batch, int n,
     int doubled, uint32_t q1, const cplx* __restrict__ bskf, FFTTables Tg,
     uint32_t* __restrict__ lweN, int logf, const uint32_t* __restrict__ tv) {
     constexpr int N = GATE_N, M = N / 2;
-    __shared__ cplx lds_all[4][FFT512_LDS_CPLX];
-    __shared__ uint16_t at_all[4][1024];
-    __shared__ cplx tw_lds[1024];
+    __shared__ cplx lds_all[4][PAIR_LDS_CPLX];
+    __shared__ cplx tab[PAIR_TABLE_CPLX];
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t cidx = blockIdx.x * 4 + w;
-    // twiddle tables staged in LDS: per-lane table reads through the vector memory
-    // path stall the FFT passes far more than LDS reads do
-    for (int k = threadIdx.x; k < 512; k += blockDim.x) {
-        tw_lds[k] = Tg.p1t[k];
-        tw_lds[512 + k] = Tg.p2[k];
-    }
+    for (int k = threadIdx.x; k < PAIR_TABLE_CPLX; k += blockDim.x) tab[k] = Tg.pair[k];
     __syncthreads();
-    const FFTTables T{tw_lds, tw_lds + 512, Tg.rot};
     if (cidx >= batch) return;
-    cplx* lds = lds_all[w];
-    uint16_t* at = at_all[w];
+    const PairAddr A(lds_all[w], lane);
     const uint32_t* c1 = ct1 + (size_t)cidx * (n + 1);
+    const uint32_t* c2 = FUNC ? nullptr : ct2 + (size_t)cidx * (n + 1);
     constexpr int LOG2N2 = 11;
-    const uint32_t q = 2u * N;
-    uint32_t acc[2][16];
-    if constexpr (FUNC) {
-        const uint32_t cmask = (q >> logf) - 1u;
-        for (int k = lane; k < n; k += 64) at[k] = (uint16_t)((c1[k] & cmask) << logf);
-        const uint32_t b = c1[n] & cmask;
-        const uint32_t fmask = (1u << logf) - 1u;
+    constexpr uint32_t q = 2u * N;
+    // digits by the offset method: with OFF added (the accumulator is kept that way) and the top
+    // bit of each digit flipped, digit j is bits [sh, sh + LOGB) sign-extended
+    constexpr uint32_t OFF = digit_offset32<GATE_LOGB, GATE_L>();
+    constexpr int IGN = 32 - GATE_L * GATE_LOGB;
+    uint32_t flip = 0;
 #pragma unroll
-        for (int s = 0; s < 16; ++s) {
-            const uint32_t c = (uint32_t)(64 * s + lane);  // < N, so j = c >> logf < ctmod / 2
-            acc[0][s] = 0u;
-            acc[1][s] = (c & fmask) ? 0u : tv[(b - (c >> logf)) & cmask];
-        }
-    } else {
-        const uint32_t* c2 = ct2 + (size_t)cidx * (n + 1);
-        for (int k = lane; k < n; k += 64) {
-            uint32_t v = c1[k] + c2[k];
-            if (doubled) v *= 2u;
-            at[k] = (uint16_t)modswitch_2N(v, LOG2N2);
-        }
-        uint32_t vb = c1[n] + c2[n];
-        if (doubled) vb *= 2u;
-        const uint32_t bt = modswitch_2N(vb, LOG2N2);
+    for (int j = 0; j < GATE_L; ++j) flip |= 1u << (IGN + (j + 1) * GATE_LOGB - 1);
+    // half u = lane >> 5 holds polynomial u: coefficients 32 a + d (re) and + 512 (im)
+    const int u = lane >> 5, d = lane & 31;
+    uint32_t re[16], im[16];
+    {
+        uint32_t bt;
+        const uint32_t cmask = FUNC ? (q >> logf) - 1u : 0u, fmask = FUNC ? (1u << logf) - 1u : 0u;
         const uint32_t q2 = (q1 + N) & (q - 1);
+        if constexpr (FUNC) {
+            bt = c1[n] & cmask;
+        } else {
+            uint32_t vb = c1[n] + c2[n];
+            if (doubled) vb *= 2u;
+            bt = modswitch_2N(vb, LOG2N2);
+        }
+        auto start = [&](uint32_t c) -> uint32_t {
+            if (!u) return 0u;
+            if constexpr (FUNC) return (c & fmask) ? 0u : tv[(bt - (c >> logf)) & cmask];
+            else return gate_tv(q1, q2, bt, c, q);
+        };
 #pragma unroll
-        for (int s = 0; s < 16; ++s) {
-            acc[0][s] = 0u;
-            acc[1][s] = gate_tv(q1, q2, bt, (uint32_t)(64 * s + lane), q);
+        for (int a = 0; a < 16; ++a) {
+            re[a] = start((uint32_t)(32 * a + d)) + OFF;
+            im[a] = start((uint32_t)(32 * a + d + M)) + OFF;
         }
     }
-    wave_sync();
+    const uint32_t kat = (uint32_t)lane * sizeof(cplx);
+    const double magic = round_magic();
+    // evaluation exponent of this lane's product frequencies at p = 0
+    const uint32_t e0 = 1u + 4u * rev_bits((uint32_t)(lane & 15), 4) + 512u * ((lane >> 4) & 1) + 1024u * (lane >> 5);
 
-    for (int i = 0; i < n; ++i) {
-        const uint32_t mrot = (q - (uint32_t)at[i]) & (q - 1);
-        if (mrot == 0) continue;
-        const cplx* key = bskf + (size_t)i * GATE_ROWS * 2 * M;
-        cplx macc[2][8];
-#pragma unroll
-        for (int o = 0; o < 2; ++o)
-#pragma unroll
-            for (int f = 0; f < 8; ++f) macc[o][f] = {0.0, 0.0};
-
-        constexpr uint32_t OFF = digit_offset32<GATE_LOGB, GATE_L>();
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            uint32_t tp[16];
-#pragma unroll
-            for (int s = 0; s < 16; ++s) tp[s] = acc[u][s] + OFF;
+    for (int i0 = 0; i0 < n; i0 += 64) {
+        // 64 steps' rotations, one per lane
+        uint32_t av = 0;
+        if (i0 + lane < n) {
+            if constexpr (FUNC) {
+                av = (c1[i0 + lane] & ((q >> logf) - 1u)) << logf;
+            } else {
+                uint32_t v = c1[i0 + lane] + c2[i0 + lane];
+                if (doubled) v *= 2u;
+                av = modswitch_2N(v, LOG2N2);
+            }
+        }
+        const int cnt = n - i0 < 64 ? n - i0 : 64;
+        for (int i = 0; i < cnt; ++i) {
+            const uint32_t mrot = (q - (uint32_t)__builtin_amdgcn_readlane((int)av, i)) & (q - 1);
+            if (mrot == 0) continue;
+            const cplx* key = bskf + (size_t)(i0 + i) * GATE_ROWS * 2 * M;
+            cplx macc[2][8];
 #pragma unroll
             for (int j = 0; j < GATE_L; ++j) {
-                const int r = 2 * j + u;
-                cplx x[8];
+                cplx x[16];
+                const int sh = IGN + j * GATE_LOGB;
 #pragma unroll
-                for (int a = 0; a < 8; ++a)
-                    x[a] = {(double)digit32<GATE_LOGB, GATE_L>(tp[a], j),
-                            (double)digit32<GATE_LOGB, GATE_L>(tp[a + 8], j)};
-                fft512_fwd(x, lds, T, lane);
-                const cplx* kr = key + (size_t)r * 2 * M;
+                for (int a = 0; a < 16; ++a)
+                    x[a] = {(double)((int32_t)((re[a] ^ flip) << (32 - sh - GATE_LOGB)) >> (32 - GATE_LOGB)),
+                            (double)((int32_t)((im[a] ^ flip) << (32 - sh - GATE_LOGB)) >> (32 - GATE_LOGB))};
+                fft512_pair_fwd(x, A, tab, lane);
+                // both polynomials' rows at 8 frequencies per lane: x[2p] is row 2j, x[2p + 1] row
+                // 2j + 1.  Key values in batches of 4 (half a row for one output), KD in flight
+                // (left to itself the compiler waits for each load in turn)
+                constexpr int KD = 3;
+                cplx kv[KD][4];
+                auto load = [&](int t) {  // batch t: row t / 4, output (t / 2) % 2, p = 4 (t % 2) ..
+                    const uint32_t at = fresh_offset(kat);
+#pragma unroll
+                    for (int p = 0; p < 4; ++p)
+                        kv[t % KD][p] = key_at(key + (4 * j + t / 2) * M + (4 * (t & 1) + p) * 64, at);
+                };
+#pragma unroll
+                for (int t = 0; t < KD; ++t) load(t);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int p = 0; p < 8; ++p) swap_rows32(x[2 * p], x[2 * p + 1]);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const int r = t / 4, o = (t / 2) & 1, s0 = 4 * (t & 1);
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {
+                        if (j == 0 && r == 0) macc[o][s0 + p] = cmul(x[2 * (s0 + p)], kv[t % KD][p]);
+                        else cmac(macc[o][s0 + p], x[2 * (s0 + p) + r], kv[t % KD][p]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (t + KD < 8) load(t + KD);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // CGGI monic update acc += (X^m - 1) t in the Fourier domain: the value at w^e is
+            // multiplied by w^(m e) - 1; one rounding of (X^m - 1) t gives the same integers as
+            // rotating the rounded t.  One table lookup per lane (a gather of one cache line per
+            // lane), turned by the powers of w^(64 m) for the p of a lane
+            {
+                const cplx z0 = Tg.rot[(mrot * e0) & (q - 1)];
+                const cplx g1 = key_at(Tg.rot, ((64u * mrot) & (q - 1)) * (uint32_t)sizeof(cplx));
+                const cplx g2 = key_at(Tg.rot, ((128u * mrot) & (q - 1)) * (uint32_t)sizeof(cplx));
+                const cplx g3 = key_at(Tg.rot, ((256u * mrot) & (q - 1)) * (uint32_t)sizeof(cplx));
+                cplx z[8];  // p = 4 b5 + 2 b6 + b7: exponent + 64 b5 + 128 b6 + 256 b7
+                z[0] = z0;
+                z[4] = cmul(z0, g1);
+                z[2] = cmul(z0, g2);
+                z[6] = cmul(z[4], g2);
+#pragma unroll
+                for (int p = 0; p < 8; p += 2) z[p + 1] = cmul(z[p], g3);
 #pragma unroll
                 for (int o = 0; o < 2; ++o)
 #pragma unroll
-                    for (int f = 0; f < 8; ++f) cmac(macc[o][f], x[f], kr[(o * 8 + f) * 64 + lane]);
+                    for (int p = 0; p < 8; ++p) macc[o][p] = cmul(macc[o][p], {z[p].re - 1.0, z[p].im});
             }
-        }
-
-        // CGGI monic update acc += (X^m - 1) t in the Fourier domain: X[k] is the
-        // polynomial at zeta_k = w^(1 - 4k), so X^m multiplies it by w^(m (1 - 4k));
-        // one rounding of (X^m - 1) t gives the same integers as rotating the rounded t
-        cplx rf[8];
-        {
-            const uint32_t kl = (uint32_t)((lane >> 3) + 8 * (lane & 7));  // k = kl + 64 f
+            // output o to half o
+            cplx x[16];
 #pragma unroll
-            for (int f = 0; f < 8; ++f) {
-                const uint32_t k = kl + 64u * f;
-                const uint32_t ex = (mrot * ((2u * N + 1u - 4u * k) & (2u * N - 1u))) & (2u * N - 1u);
-                const cplx r = T.rot[ex];
-                rf[f] = {r.re - 1.0, r.im};
+            for (int p = 0; p < 8; ++p) {
+                x[2 * p] = macc[0][p];
+                x[2 * p + 1] = macc[1][p];
+                swap_rows32(x[2 * p], x[2 * p + 1]);
             }
-        }
+            fft512_pair_inv(x, A, tab, lane);
 #pragma unroll
-        for (int o = 0; o < 2; ++o) {
-            cplx x[8];
-#pragma unroll
-            for (int f = 0; f < 8; ++f) x[f] = cmul(macc[o][f], rf[f]);
-            fft512_inv(x, lds, T, lane);
-#pragma unroll
-            for (int a = 0; a < 8; ++a) {
-                acc[o][a] += round_mod32(x[a].re, 1.0 / M);
-                acc[o][a + 8] += round_mod32(x[a].im, 1.0 / M);
+            for (int a = 0; a < 16; ++a) {
+                re[a] += round_mod32(x[a].re, 1.0 / M, magic);
+                im[a] += round_mod32(x[a].im, 1.0 / M, magic);
             }
         }
     }
 
+    const int d1 = fresh_lane(d);
     // sample extraction at coefficient 0 (X -> X^{2N-1} automorphism, bitwise/src/kernel.cu:241-250)
     uint32_t* out = lweN + (size_t)cidx * (N + 1);
+    if (!u) {
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
-        const int c = 64 * s + lane;
-        const uint32_t v = acc[0][s];
-        out[(N - c) & (N - 1)] = c ? 0u - v : v;
+        for (int a = 0; a < 16; ++a) {
+            const int c = 32 * a + d1;
+            const uint32_t v = re[a] - OFF;
+            out[(N - c) & (N - 1)] = c ? 0u - v : v;
+            out[N - c - M] = OFF - im[a];
+        }
+    } else if (d == 0) {
+        out[N] = FUNC ? re[0] - OFF : re[0] - OFF + (1u << 29) + 1u;
     }
-    if (lane == 0) out[N] = FUNC ? acc[1][0] : acc[1][0] + (1u << 29) + 1u;
 }
 
 // ===========================================================================
@@ -286,6 +328,13 @@ __global__ __launch_bounds__(256) void k_gate_blind_rotate(
 // Three barriers per step.  Every rounding gives the exact integers of the batched form.
 // ===========================================================================
 constexpr int GSPLIT_WAVES = 2 * GATE_ROWS;
+
+// place of the 256-point step's lane 16 k0 + 4 e + p in a 64-entry LDS block: eight
+// neighbouring lanes touch all banks both in this order and in the key's (bit-reversed) order
+__device__ __forceinline__ int split_pos(int lane) {
+    const int k0 = lane >> 4, e = (lane >> 2) & 3, p = lane & 3;
+    return ((e | ((k0 & 2) << 1)) ^ (p << 1)) + 8 * ((k0 & 1) + 2 * p);
+}
 
 template <bool FUNC>
 __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_split(
@@ -307,13 +356,19 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
     const bool inv = w < 4;                                        // inverse role: output w >> 1, half r
     const int iv = (w >> 1) & 1;
     const int f = (w - 4) >> 1, o = w & 1;                         // product role (w >= 4)
-    // the key's frequency lane 8 k0 + e holds k = 64 f + k0 + 8 e; the 256-point step leaves
-    // k = k0' + 4 e' + 16 p' + 64 s at slot s of lane 16 k0' + 4 e' + p'
-    const int kk = (lane >> 3) + 8 * (lane & 7);
-    const int pos = f * 64 + 16 * (kk & 3) + 4 * ((kk >> 2) & 3) + (kk >> 4);
-    const uint32_t ek = (1u - 4u * (uint32_t)(kk + 64 * f)) & (q - 1u);
-    const uint32_t kat = (uint32_t)(o * M + f * 64 + lane) * sizeof(cplx);
-    const cplx cross = Tg.two[768 + (f & 3) * 64 + lane];
+    // product lane (n, b8, x) holds the frequency at key positions p = 2 f + x, lane n + 16 b8 and
+    // + 32 (pair_pos): k mod 256 = -K0, K0 = rev(n) + 16 rev(p) + 128 b8, b9 = 0 giving k itself
+    // only for K0 = 0.  The 256-point step leaves k = k0 + 4 e + 16 p + 64 s at slot s of lane
+    // 16 k0 + 4 e + p
+    const int pp = 2 * (f & 3) + (lane >> 5);
+    const uint32_t K0 = rev_bits((uint32_t)(lane & 15), 4) + 16u * rev_bits((uint32_t)pp, 3) + 128u * ((lane >> 4) & 1);
+    const int kk = (int)((256u - K0) & 255u);
+    const int pos = 64 * (kk >> 6) + split_pos(16 * (kk & 3) + 4 * ((kk >> 2) & 3) + ((kk >> 4) & 3));
+    const int lpos = split_pos(lane);
+    const uint32_t ek = (1u - 4u * (uint32_t)kk) & (q - 1u);
+    const uint32_t kat = (uint32_t)(o * M + pp * 64 + (lane & 31)) * sizeof(cplx);  // b9 = 0
+    const uint32_t kat0 = kat + (K0 ? 32 * sizeof(cplx) : 0), kat1 = kat + (K0 ? 0 : 32 * sizeof(cplx));
+    const cplx cross = Tg.two[768 + kk];
     for (int k = threadIdx.x; k < 2 * N; k += blockDim.x) rot[k] = Tg.rot[k];
     for (uint32_t cidx = blockIdx.x; cidx < batch; cidx += gridDim.x) {
         const uint32_t* c1 = ct1 + (size_t)cidx * (n + 1);
@@ -364,7 +419,7 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
                         (double)((int32_t)(((vi[a] + OFF) >> sh) & BM) - HB)};
             fft256_fwd(x, bufs[w], T, lane);
 #pragma unroll
-            for (int s = 0; s < 4; ++s) bufs[w][s * 64 + lane] = x[s];
+            for (int s = 0; s < 4; ++s) bufs[w][s * 64 + lpos] = x[s];
         };
         // two loops with the same barriers: merged, the key values in flight would be moved
         // (and waited for) where the roles' paths join
@@ -372,10 +427,11 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
             cplx kv[GATE_ROWS][2];  // key values of k and k + 256
             auto load_keys = [&](int i) {
                 const cplx* key = bskf + (size_t)i * GATE_ROWS * 2 * M;
+                const uint32_t a0 = fresh_offset(kat0), a1 = fresh_offset(kat1);
 #pragma unroll
                 for (int t = 0; t < GATE_ROWS; ++t) {
-                    kv[t][0] = key_at(key + t * 2 * M, kat);
-                    kv[t][1] = key_at(key + t * 2 * M + 256, kat);
+                    kv[t][0] = key_at(key + t * 2 * M, a0);
+                    kv[t][1] = key_at(key + t * 2 * M, a1);
                 }
             };
             load_keys(0);
@@ -411,7 +467,7 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
                 lds_barrier();
                 cplx x[4];
 #pragma unroll
-                for (int s = 0; s < 4; ++s) x[s] = prod[iv][r][s * 64 + lane];
+                for (int s = 0; s < 4; ++s) x[s] = prod[iv][r][s * 64 + lpos];
                 fft256_inv(x, bufs[w], T, lane);
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
@@ -465,12 +521,16 @@ __global__ __launch_bounds__(64) void k_plain_mac_ifft(const cplx* __restrict__ 
     __shared__ cplx lds[FFT512_LDS_CPLX];
     const int lane = threadIdx.x, o = blockIdx.x;
     cplx x[8];
+    uint32_t kpos[8];  // the key's positions of this lane's frequencies
 #pragma unroll
-    for (int f = 0; f < 8; ++f) x[f] = {0.0, 0.0};
+    for (int f = 0; f < 8; ++f) {
+        x[f] = {0.0, 0.0};
+        kpos[f] = pair_pos((uint32_t)((lane >> 3) + 8 * (lane & 7) + 64 * f));
+    }
     for (int r = 0; r < GATE_ROWS; ++r)
 #pragma unroll
         for (int f = 0; f < 8; ++f)
-            cmac(x[f], digf[(r * 8 + f) * 64 + lane], key[((r * 2 + o) * 8 + f) * 64 + lane]);
+            cmac(x[f], digf[(r * 8 + f) * 64 + lane], key[(r * 2 + o) * 512 + kpos[f]]);
     fft512_inv(x, lds, T, lane);
 #pragma unroll
     for (int a = 0; a < 8; ++a) {

@@ -68,6 +68,7 @@ struct PbsStep {
     // offset: scalar base addresses, one vector offset for all loads
     static __device__ __forceinline__ void load(cplx (&kv)[2][4], const cplx* key, uint32_t at, int u, int t,
                                                 int first, int second) {
+        at = fresh_offset(at);
         const int j = t / BPR, b = t % BPR, r = 2 * j + u;
 #pragma unroll
         for (int o = 0; o < 2; ++o) {
@@ -375,6 +376,7 @@ struct PbsPair {
     cplx fp[2][S::FP][NQ];
 
     static __device__ __forceinline__ void load(cplx (&kv)[4], const cplx* key, uint32_t at, int u, int t) {
+        at = fresh_offset(at);
         const int j = t / S::BPR, b = t % S::BPR, r = 2 * j + u;
 #pragma unroll
         for (int o = 0; o < 2; ++o) {
