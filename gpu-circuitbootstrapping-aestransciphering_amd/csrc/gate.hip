@@ -855,12 +855,14 @@ unsigned device_cus() {
 
 int ks_model_slices(uint32_t batch, int N, int n) {
     // i-slices: as many workgroups as run at once (two per CU: 100 VGPRs and 8 waves
-    // each), so the launch is one full round; each slice >= 32 coefficients, with one or two
-    // ciphertext groups >= 8: there a workgroup's time is its slice's chain of key loads
-    // (N = 1024, 1 / 61 / 200 ciphertexts: 0.115 / 0.125 / 0.150 ms with 32, 0.051 / 0.073 / 0.129 with 8;
-    // three groups 0.166 against 0.174)
+    // each), so the launch is one full round; each slice >= 32 coefficients, of the gate level's
+    // N = 1024 with one or two ciphertext groups >= 8: there a workgroup's time is its slice's
+    // chain of key loads (1 / 61 / 200 ciphertexts: 0.115 / 0.125 / 0.150 ms with 32,
+    // 0.051 / 0.073 / 0.129 with 8; three groups 0.166 against 0.174).  N = 2048 keeps 32 (at most
+    // the 64 slices that tfhe_cbs_autotune chooses from; 128 ciphertexts 0.184 against 0.148 ms
+    // of a round that takes over 9)
     const unsigned cols = (unsigned)(n + 1 + 127) / 128, groups = ks_bpad(batch) / KS_GROUP;
-    const unsigned slots = 2 * device_cus(), least = groups <= 2 ? 8 : 32;
+    const unsigned slots = 2 * device_cus(), least = groups <= 2 && N <= 1024 ? 8 : 32;
     unsigned slices = slots / (cols * groups);
     if (slices > (unsigned)N / least) slices = (unsigned)N / least;
     if (slices < 1) slices = 1;
