@@ -510,18 +510,24 @@ __global__ __launch_bounds__(256) void k_htss(const uint64_t* __restrict__ acc_i
 //
 // k_pfks_digits rounds the inputs and transposes them to [i][Bpad] so that
 // one i-row of a wave's PF_CT inputs is a uniform (scalar-load) read.
-// k_pfks32: a workgroup of PF_WAVES waves shares one 128-column tile of the
-// key; per (i, t) the 15 candidate rows are loaded once by the workgroup into
-// an LDS table (row 0 = 0, double-buffered, one barrier per step) and every
-// wave selects, for each of its PF_CT inputs, the row named by that input's
-// digit: one LDS read and one subtraction per (input, column).  blockIdx.z
-// picks an i-slice and the function; slices add into the zero-filled output
-// with 32-bit atomics (addition mod 2^32 is order-free, so the result is
-// exact).  The key is read once per (column tile, input group) from L2, and
-// the workgroups of one key tile share an XCD (their linear ids differ by
-// multiples of 64), so HBM sees it about once.
+// k_pfks32: a workgroup of 16 waves shares a 128- or 256-column tile of the key; per (i, t) the 15
+// candidate rows go straight from memory into a ring in LDS (three pairs of rows' tiles in
+// flight, one barrier per pair).  A wave keeps the step's 16 rows of its 128 columns in
+// registers and subtracts, for each of its 32 inputs, the row that the digit names: the
+// register index comes from the scalar digit (s_set_gpr_idx), so a row is read from LDS once per
+// 32 inputs.  (Selecting the rows in LDS, one 8-byte read per input, lane and digit, ran at the
+// LDS bandwidth: 4 bytes per subtraction.)  Bound by the key's 8.06 GB up to 256 inputs, above by
+// the issue of the indexed subtractions (2.0 ns per instruction and SIMD against 1.3 for plain
+// ones) and the LDS reads of the rows, which are half overlapped; 8 waves of 64 inputs with the
+// next rows read during the subtractions, or of 32 inputs x 4 columns, took the same time at 512
+// inputs and 0.2 ms more at 16.  Both functions, ms before / after: 16 inputs 1.36 / 1.28, 256
+// 2.11 / 1.85, 320 4.26 / 2.79, 512 4.16 / 3.40, 2560 21.8 / 19.7.
+// blockIdx.z picks an i-slice and the function; slices add into the zero-filled output with 32-bit
+// atomics (addition mod 2^32 is order-free, so the result is exact).  The workgroups of one key
+// tile share an XCD's L2 (their linear ids differ by multiples of 16), so HBM sees the key about
+// once.
 // ===========================================================================
-constexpr int PF_WAVES = 8, PF_CT = 32, PF_GROUP = PF_WAVES * PF_CT;
+constexpr int PF_WAVES = 16, PF_CT = 32, PF_PAD = 256;
 
 __global__ __launch_bounds__(256) void k_pfks_digits(const uint64_t* __restrict__ lwe64, uint32_t B, uint32_t Bpad,
                                                     uint32_t* __restrict__ at) {
@@ -544,12 +550,50 @@ __global__ __launch_bounds__(256) void k_pfks_digits(const uint64_t* __restrict_
     }
 }
 
-__global__ __launch_bounds__(64 * PF_WAVES) void k_pfks32(const uint32_t* __restrict__ at, uint32_t B, uint32_t Bpad,
-                                                         const uint32_t* __restrict__ key, size_t key_u_stride,
-                                                         int u0, int slices, uint32_t* __restrict__ out,
-                                                         size_t out_stride, size_t out_u_offset) {
-    // two adjacent columns per lane: one LDS address and one 8-byte read feed two subtractions
-    __shared__ uint2 tab[2][16][64];
+// k_pfks32's inner block, one step of a wave: reads the tile's 15 rows (two columns per lane, row v
+// into v[32 + 2 v : 33 + 2 v], row 0 zero) and subtracts for each of 32 inputs the row that its digit
+// names (sums of input k in v[64 + 2 k : 65 + 2 k]; s[BASE + k] holds the register offsets 2 * digit
+// in byte SHIFT / 8).  The reads are waited for in the block, so nothing is in flight when it ends.
+#define PF_STEP(BASE, SHIFT)                                                                                       \
+    "v_mov_b32 v32, 0\n v_mov_b32 v33, 0\n"                                                                         \
+    ".set pf_r, 0\n .rept 15\n ds_read_b64 v[34 + 2 * pf_r : 35 + 2 * pf_r], %6 offset:%7 * pf_r\n"                 \
+    " .set pf_r, pf_r + 1\n .endr\n s_waitcnt lgkmcnt(0)\n"                                                         \
+    "s_lshr_b32 s30, s[" #BASE "], " #SHIFT "\n s_set_gpr_idx_on s30, 1\n"                                          \
+    ".set pf_k, 0\n .rept 32\n"                                                                                     \
+    " s_lshr_b32 s31, s[" #BASE " + pf_k], " #SHIFT "\n s_set_gpr_idx_idx s31\n"                                    \
+    " v_subrev_u32 v[64 + 2 * pf_k], v32, v[64 + 2 * pf_k]\n"                                                       \
+    " v_subrev_u32 v[65 + 2 * pf_k], v33, v[65 + 2 * pf_k]\n"                                                       \
+    " .set pf_k, pf_k + 1\n .endr\n s_set_gpr_idx_off\n"
+typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x32 __attribute__((ext_vector_type(32)));
+#define PF_ASM(BASE, SHIFT)                                                                                         \
+    asm volatile(PF_STEP(BASE, SHIFT)                                                                               \
+                 : "+{v[64:95]}"(acc[0]), "+{v[96:127]}"(acc[1])                                                    \
+                 : "{s[32:47]}"(x0), "{s[48:63]}"(x1), "{s[64:79]}"(y0), "{s[80:95]}"(y1), "v"(addr), "n"(512 * H)    \
+                 : "m0", "scc", "s30", "s31", "memory", "v32", "v33", "v34", "v35", "v36", "v37", "v38", "v39", "v40", \
+                   "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52", "v53", "v54",  \
+                   "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63")
+
+// 16 bytes per lane from memory into LDS, lane l at dst + 16 l
+__device__ __forceinline__ void load_lds16(const char* src, uint4* dst) {
+    __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) const void*)src,
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+// all but this wave's last LOADS loads are in LDS, for every wave, and every wave is past its reads
+template <int LOADS>
+__device__ __forceinline__ void pf_sync() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// H: column halves of 128 of a workgroup's tile; it covers 16 / H * 32 inputs
+template <int H>
+__global__ __launch_bounds__(64 * PF_WAVES, 1) void k_pfks32(const uint32_t* __restrict__ at, uint32_t B, uint32_t Bpad,
+                                                            const uint32_t* __restrict__ key, size_t key_u_stride,
+                                                            int u0, int slices, uint32_t* __restrict__ out,
+                                                            size_t out_stride, size_t out_u_offset) {
+    __shared__ uint4 tab[4][2][16][32 * H];  // row 15 is never read
     constexpr int N = CB_N, COLS = 2 * CB_N;
     const int ISLICE = (N + 1 + slices - 1) / slices;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -559,73 +603,67 @@ __global__ __launch_bounds__(64 * PF_WAVES) void k_pfks32(const uint32_t* __rest
     const int ibeg = slice * ISLICE;
     const int iend = (ibeg + ISLICE) < (N + 1) ? (ibeg + ISLICE) : (N + 1);
     if (ibeg >= iend) return;  // empty slice (uniform over the workgroup)
-    const uint32_t cbase = blockIdx.y * PF_GROUP + w * PF_CT;
-    const bool active = cbase < B;  // idle waves still take part in the barriers
-    // this thread's share of a tile: candidate v = 1 + w (all waves) and v = 9 + w (waves 0..6)
-    const uint2* kcol = reinterpret_cast<const uint2*>(key + (size_t)u * key_u_stride + blockIdx.x * 128) + lane;
-    const bool second = w < 7;
-    if (tid < 64) {
-        tab[0][0][tid] = make_uint2(0, 0);
-        tab[1][0][tid] = make_uint2(0, 0);
-    }
-    uint32_t acc[PF_CT][2];
+    const int half = H == 2 ? w & 1 : 0;
+    const uint32_t cbase = blockIdx.y * (PF_WAVES / H * PF_CT) + (w / H) * PF_CT;
+    const bool active = cbase < B;  // idle waves still take part in the loads and barriers
+    // Loads of 1 KB: H = 2: row v = 1 + w of both tiles of a pair; H = 1: rows 1 + r and 2 + r,
+    // r = 2 (w & 7), of tile w >> 3.  (Row 16 does not exist: row 15 again, so that every wave has
+    // the same number of loads in flight.)
+    const int row = H == 2 ? w : 2 * (w & 7) + (lane >> 5);
+    const char* kcol = reinterpret_cast<const char*>(key + (size_t)u * key_u_stride + blockIdx.x * (128 * H)) +
+                       (size_t)(row < 15 ? row : 14) * (COLS * 4) + (H == 2 ? lane : lane & 31) * 16;
+    // Tiles come in pairs, four to a coefficient.  Pair p = 4 (i - ibeg) + tp goes straight from
+    // memory into tab[p & 3], issued at the start of pair p - 3: three pairs are in flight.
+    auto load_pair = [&](int slot, int i, int tp) {
+        const int il = i < iend ? i : iend - 1;  // past the end: loaded, never read
 #pragma unroll
-    for (int k = 0; k < PF_CT; ++k) acc[k][0] = acc[k][1] = 0;
-    // Tile m (m = 8 (i - ibeg) + t) is loaded into register slot m % PF_RING at step
-    // m - PF_RING, stored into tab[m & 1] at the start of step m - 1 and read at step m:
-    // PF_RING - 1 steps of latency cover the key stream.  With the t loop unrolled by 8
-    // every slot index is a compile-time constant.
-    constexpr int PF_RING = 4;
-    uint2 kv[PF_RING][2];
-    auto load_tile = [&](int slot, int i, int t) {
-        uint64_t off = ((uint64_t)(i * 8 + t) * 15 + w) * (COLS / 2);
-        asm volatile("" : "+s"(off));  // keep the prefetch where it is written
-        const uint2* kr = kcol + off;
-        kv[slot][0] = kr[0];
-        kv[slot][1] = second ? kr[(size_t)8 * (COLS / 2)] : make_uint2(0, 0);
-    };
-    auto store_tile = [&](int slot, int b) {
-        tab[b][1 + w][lane] = kv[slot][0];
-        if (second) tab[b][9 + w][lane] = kv[slot][1];
+        for (int l = 0; l < H; ++l) {
+            const int h = H == 2 ? l : w >> 3;
+            load_lds16(kcol + (size_t)(il * 8 + 2 * tp + h) * 15 * (COLS * 4), &tab[slot][h][H == 2 ? w : 2 * (w & 7)][0]);
+        }
     };
 #pragma unroll
-    for (int m = 0; m < PF_RING; ++m)
-        if (ibeg + m / 8 < iend) load_tile(m, ibeg + m / 8, m % 8);
-    store_tile(0, 0);
-    __syncthreads();
+    for (int p = 0; p < 3; ++p) load_pair(p, ibeg, p);
+    pf_sync<2 * H>();
+    const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint4*)&tab[0][0][0][0] +
+                          (uint32_t)(half * 512 + lane * 8);
+    u32x32 acc[2] = {};
     for (int i = ibeg; i < iend; ++i) {
-        uint32_t a[PF_CT];
-        if (active) {
-            const uint32_t* ar = at + (size_t)i * Bpad + cbase;
-#pragma unroll
-            for (int k = 0; k < PF_CT; ++k) a[k] = ar[k];
+        u32x16 x0, x1, y0, y1;  // 2 * digit in bytes: even digits (x), odd digits (y) of inputs 0..15, 16..31
+        {
+            const u32x16* ar = reinterpret_cast<const u32x16*>(at + (size_t)i * Bpad + (active ? cbase : 0));
+            const u32x16 a0 = ar[0], a1 = ar[1];
+            x0 = (a0 << 1) & 0x1e1e1e1eu;
+            x1 = (a1 << 1) & 0x1e1e1e1eu;
+            y0 = (a0 >> 3) & 0x1e1e1e1eu;
+            y1 = (a1 >> 3) & 0x1e1e1e1eu;
         }
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            // store tile m + 1 (loaded PF_RING - 1 steps ago), refill its slot with tile m + PF_RING
-            const int t1 = t + 1, tr = t + PF_RING;
-            if (i + t1 / 8 < iend) store_tile(t1 % PF_RING, t1 & 1);
-            if (i + tr / 8 < iend) load_tile(tr % PF_RING, i + tr / 8, tr % 8);
+        for (int tp = 0; tp < 4; ++tp) {
+            load_pair((tp + 3) & 3, i + (tp + 3) / 4, (tp + 3) & 3);
             if (active) {
-#pragma unroll
-                for (int k = 0; k < PF_CT; ++k) {
-                    const uint2 v = tab[t & 1][(a[k] >> (4 * t)) & 15u][lane];
-                    acc[k][0] -= v.x;
-                    acc[k][1] -= v.y;
-                }
+                uint32_t addr = base + (uint32_t)tp * sizeof(tab[0]);
+                if (tp == 0) PF_ASM(32, 0);
+                if (tp == 1) PF_ASM(32, 8);
+                if (tp == 2) PF_ASM(32, 16);
+                if (tp == 3) PF_ASM(32, 24);
+                addr += sizeof(tab[0][0]);
+                if (tp == 0) PF_ASM(64, 0);
+                if (tp == 1) PF_ASM(64, 8);
+                if (tp == 2) PF_ASM(64, 16);
+                if (tp == 3) PF_ASM(64, 24);
             }
-#pragma unroll
-            for (int k = 0; k < PF_CT; ++k) asm volatile("" : "+v"(acc[k][0]), "+v"(acc[k][1]));
-            __syncthreads();
+            pf_sync<2 * H>();
         }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the loads past the end
     if (active) {
-        uint32_t* o = out + (size_t)(u - u0) * out_u_offset + blockIdx.x * 128 + 2 * lane;
+        uint32_t* o = out + (size_t)(u - u0) * out_u_offset + blockIdx.x * (128 * H) + 128 * half + 2 * lane;
 #pragma unroll
         for (int k = 0; k < PF_CT; ++k)
             if (cbase + k < B) {
-                atomicAdd(&o[(size_t)(cbase + k) * out_stride], acc[k][0]);
-                atomicAdd(&o[(size_t)(cbase + k) * out_stride + 1], acc[k][1]);
+#pragma unroll
+                for (int c = 0; c < 2; ++c) atomicAdd(&o[(size_t)(cbase + k) * out_stride + c], acc[k / 16][2 * (k % 16) + c]);
             }
     }
 }
@@ -1339,7 +1377,11 @@ void launch_xor_public(uint32_t* ct, const uint8_t* pub, uint32_t nbits, int n, 
     k_xor_public<<<(nbits + 255) / 256, 256, 0, st>>>(ct, pub, nbits, n);
 }
 
-uint32_t pfks_bpad(uint32_t B) { return (B + PF_GROUP - 1) / PF_GROUP * PF_GROUP; }
+uint32_t pfks_bpad(uint32_t B) { return (B + PF_PAD - 1) / PF_PAD * PF_PAD; }
+// Column halves per workgroup: at most 256 inputs take 256-column tiles (whole 1 KB rows of the key
+// per load), more take 512 inputs x 128 columns, so that the key is read once for all of them
+// (512 inputs: 3.40 ms against 3.49 in two groups of 256; 320: 2.79 against 3.4)
+static int pfks_halves(uint32_t B) { return B <= 256 ? 2 : 1; }
 
 void launch_pfks_digits(const uint64_t* lwe64, uint32_t B, uint32_t* at, hipStream_t st) {
     const uint32_t Bpad = pfks_bpad(B);
@@ -1363,11 +1405,12 @@ void launch_zero_rows32(uint32_t* out, uint32_t count, size_t stride, uint32_t w
 
 int pfks_model_slices(uint32_t B, int nu) {
     // i-slices (4..32): the launch runs in rounds of as many workgroups as fit at once
-    // (two per CU: 92 VGPRs and 8 waves each), and a workgroup's time is its slice
+    // (one of 16 waves per CU), and a workgroup's time is its slice
     // length, so pick the slice count with the fewest rounds x coefficients per
     // slice; ties go to fewer slices (each slice is one more atomic pass over the outputs)
-    const unsigned tiles = 2 * CB_N / 128, groups = pfks_bpad(B) / PF_GROUP;
-    const unsigned slots = 2 * device_cus(), per_slice = tiles * groups * (unsigned)nu;
+    const unsigned h = (unsigned)pfks_halves(B), per_group = PF_WAVES / h * PF_CT;
+    const unsigned tiles = 2 * CB_N / (128 * h), groups = (B + per_group - 1) / per_group;
+    const unsigned slots = device_cus(), per_slice = tiles * groups * (unsigned)nu;
     int slices = 4;
     unsigned long long best = ~0ull;
     for (unsigned sl = 4; sl <= 32; ++sl) {
@@ -1385,10 +1428,11 @@ void launch_pfks32(const uint32_t* at, uint32_t B, const uint32_t* key, size_t k
                    uint32_t* out, size_t out_stride, size_t out_u_offset, hipStream_t st, int slices) {
     if (slices <= 0) slices = pfks_model_slices(B, nu);
     if (slices > CB_N + 1) slices = CB_N + 1;
-    const unsigned tiles = 2 * CB_N / 128, groups = pfks_bpad(B) / PF_GROUP;
-    dim3 grid(tiles, groups, (unsigned)(slices * nu));
-    k_pfks32<<<grid, 64 * PF_WAVES, 0, st>>>(at, B, pfks_bpad(B), key, key_u_stride, u0, slices, out, out_stride,
-                                              out_u_offset);
+    const unsigned h = (unsigned)pfks_halves(B), per_group = PF_WAVES / h * PF_CT;
+    dim3 grid(2 * CB_N / (128 * h), (B + per_group - 1) / per_group, (unsigned)(slices * nu));
+    auto kernel = h == 2 ? k_pfks32<2> : k_pfks32<1>;
+    kernel<<<grid, 64 * PF_WAVES, 0, st>>>(at, B, pfks_bpad(B), key, key_u_stride, u0, slices, out, out_stride,
+                                            out_u_offset);
 }
 
 size_t pfkl_key_bytes() { return (size_t)2 * PFKL_SLICES * 2 * CB_N * PFKL_KP; }

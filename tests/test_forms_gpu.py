@@ -1,0 +1,143 @@
+"""The kernel forms that a launch's size chooses, at the sizes where one begins or a workgroup is
+partly filled: the same words as the other form's, and the oracle's on sampled inputs."""
+import numpy as np
+import pytest
+
+import oracle as O
+from conftest import from_dev, to_dev
+
+pytestmark = pytest.mark.gpu
+
+SEED = 21
+
+
+@pytest.fixture(scope="module")
+def gkeys():
+    return O.GateKeys(3)
+
+
+@pytest.fixture(scope="module")
+def gctx(gpu, gkeys):
+    import tfhe_amd
+    c = tfhe_amd.GateContext(max_batch=2048)
+    c.set_keys(gkeys.bsk, gkeys.ksk)
+    yield c
+    c.close()
+
+
+@pytest.fixture(scope="module")
+def okeys():
+    return O.CbsKeys(SEED)
+
+
+@pytest.fixture(scope="module")
+def ctx(gpu, okeys):
+    import tfhe_amd
+    c = tfhe_amd.CbsContext(max_blocks=9)
+    c.keygen(okeys.s, SEED)
+    yield c
+    c.close()
+
+
+def _rand(shape, seed, bits=32):
+    t = np.uint32 if bits == 32 else np.uint64
+    return np.random.default_rng(seed).integers(0, 2 ** bits, shape, dtype=np.uint64).astype(t)
+
+
+@pytest.mark.parametrize("count", [1, 31, 33, 255, 256, 257, 481, 511, 512, 513, 1100])
+def test_pfks_counts(ctx, okeys, count):
+    """Lookup PFKS: 32 inputs per wave, 256 (up to 256 inputs) or 512 per workgroup.  Five inputs
+    (every digit value, the wrap of the rounding, zero, random ones) repeated over the launch:
+    each row equals the oracle's."""
+    import torch
+    base = _rand((5, 2049), 12, 64)
+    base[0, :64] = np.uint64(2 ** 64 - 2 ** 31 + 5)
+    base[1, :16] = np.array([(v * 0x11111111) << 32 for v in range(16)], np.uint64)
+    base[2] = 0
+    pick = np.arange(count) * 7 % 5
+    d_in = torch.from_numpy(base[pick].view(np.int64).copy()).to("cuda")
+    for u in (0, 1):
+        d_out = torch.full((count + 1, 4096), 7, dtype=torch.int32, device="cuda")
+        ctx.pfks_batch(u, d_in, count, 4096, d_out)
+        torch.cuda.synchronize()
+        got = from_dev(d_out)
+        want = np.stack([okeys.pfks(u, base[j]) for j in range(5)])
+        assert np.array_equal(got[:count], want[pick]), u
+        assert (got[count] == 7).all()
+
+
+@pytest.mark.parametrize("func", [False, True])
+def test_gate_forms(gctx, gkeys, func):
+    """768 gates (three rounds of one ciphertext per workgroup on 256 CUs) and 769 (four one-wave
+    ciphertexts per workgroup, the last alone): equal rows, and a ciphertext without a mask."""
+    import torch
+    n1 = gkeys.p.n + 1
+    c1, c2 = _rand((769, n1), 1), _rand((769, n1), 2)
+    c1[5] = c2[5] = 0
+    rows = {}
+    for count in (1, 768, 769):
+        first = 5 if count == 1 else 0
+        d1, d2 = to_dev(c1[first:first + count]), to_dev(c2[first:first + count])
+        d_out = torch.empty((count, n1), dtype=torch.int32, device="cuda")
+        if func:
+            lut = np.repeat(np.arange(4, dtype=np.uint32) * 256, 256)
+            gctx.eval_func(to_dev(c1[first:first + count] & 1023), 1024, lut, d_out)
+        else:
+            gctx.eval_batch(O.XOR, d1, d2, d_out)
+        torch.cuda.synchronize()
+        rows[count] = from_dev(d_out)
+    assert np.array_equal(rows[768], rows[769][:768])
+    assert np.array_equal(rows[1][0], rows[768][5])
+    if not func:
+        for k in (5, 768):
+            want, _ = gkeys.bootstrap(O.XOR, c1[k], c2[k])
+            assert np.array_equal(rows[769][k], want), k
+
+
+@pytest.mark.parametrize("count", [1, 128, 129, 256, 257])
+def test_keyswitch_slices(gctx, gkeys, count):
+    """N = 1024 key switch with one, two and three ciphertext groups."""
+    import torch
+    lwe = _rand((3, gkeys.p.N + 1), 9)
+    pick = np.arange(count) % 3
+    d_out = torch.empty((count, gkeys.p.n + 1), dtype=torch.int32, device="cuda")
+    gctx.keyswitch_batch(to_dev(lwe[pick]), d_out)
+    torch.cuda.synchronize()
+    want = np.stack([O.keyswitch32(gkeys, lwe[j]) for j in range(3)])
+    assert np.array_equal(from_dev(d_out), want[pick])
+
+
+@pytest.mark.parametrize("form", ["exact", "one_bit", "two_bits", "htss"])
+def test_pbs_pairs_and_odd_batches(gpu, okeys, form):
+    """Launches above 256 inputs run two ciphertexts per workgroup (one-bit one-product: one); an
+    odd batch's last workgroup stores one.  Rows of 257 and 258 inputs agree, the row past the end
+    is untouched, and a ciphertext without a mask bootstraps as in a launch of its own (the
+    one-product forms sum in another order there, so only the exact ones compare words)."""
+    import torch
+    import tfhe_amd
+    params = {"exact": {}, "one_bit": {"pbs_approx": 1}, "two_bits": {"pbs_approx": 1, "pbs_multibit": 2},
+              "htss": {"lwe_to_rgsw": 1}}[form]
+    c = tfhe_amd.CbsContext(max_blocks=3, params=tfhe_amd.cbs_params(**params))
+    c.keygen(okeys.s, SEED)
+    cts = _rand((258, okeys.p.n + 1), 3)
+    cts[1, :-1] = 0
+    cts[2, :-1] = 0
+    cts[2, 7] = 1 << 29
+    rows = {}
+    for count in (257, 258):
+        if form == "htss":
+            d_out = torch.full((count + 1, 4, 2, 2048), 7, dtype=torch.int32, device="cuda")
+            c.cbs_batch(to_dev(cts[:count]), d_out[:count])
+        else:
+            d_out = torch.full((count + 1, 2, 2049), 7, dtype=torch.int64, device="cuda")
+            c.pbs_batch(to_dev(cts[:count]), d_out[:count])
+        torch.cuda.synchronize()
+        rows[count] = d_out.cpu().numpy()
+        assert (rows[count][count] == 7).all()
+    assert np.array_equal(rows[257][:257], rows[258][:257])
+    d_one = torch.empty_like(d_out[:3])
+    (c.cbs_batch if form == "htss" else c.pbs_batch)(to_dev(cts[:3]), d_one)
+    torch.cuda.synchronize()
+    if form in ("exact", "htss"):
+        assert np.array_equal(d_one.cpu().numpy(), rows[257][:3])
+    c.close()
