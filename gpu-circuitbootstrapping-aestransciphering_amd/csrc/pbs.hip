@@ -245,7 +245,8 @@ __device__ __forceinline__ void pbs_exponents(int w, int lane, uint32_t (&ek)[4]
 // share of the step's 128-byte lines (one word per line), issued after the step's last key
 // loads (loads return in order: earlier, the step's own key waits would include it) and
 // consumed a step later.
-template <size_t KEY_CPLX, uint32_t MAXWG, int PER>
+// (THREADS is a constant: blockDim.x would be a load from memory, and a wait for it, per step)
+template <size_t KEY_CPLX, uint32_t MAXWG, int PER, uint32_t THREADS>
 struct KeyPrefetch {
     static constexpr uint32_t LINES = KEY_CPLX * sizeof(cplx) / 128;
     uint32_t l0, end, pf[PER], sink = 0;
@@ -263,7 +264,7 @@ struct KeyPrefetch {
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
             sink ^= pf[k];  // the previous step's, long landed
-            const uint32_t l = l0 + (uint32_t)k * blockDim.x;
+            const uint32_t l = l0 + (uint32_t)k * THREADS;
             pf[k] = *reinterpret_cast<const uint32_t*>(p + (size_t)(l < end ? l : end - 1) * 128);
         }
     }
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(256, 2) void k_pbs2(const uint32_t* __restrict__ lw
     const uint32_t kat = (uint32_t)(w * 64 + lane) * sizeof(cplx);
     cplx* own = regions[w];
     constexpr uint32_t Q2 = 2 * CB_N;
-    KeyPrefetch<S::KEY, 64, 1> next;
+    KeyPrefetch<S::KEY, 64, 1, 256> next;
     for (uint32_t cidx = blockIdx.x; cidx < batch; cidx += gridDim.x) {
         __syncthreads();
         const uint32_t bt = pbs_rotations<LUT>(lwe + (size_t)cidx * (n + 1), n, at, io);
@@ -467,7 +468,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict
     cplx* group = regions[4 * cc];
     constexpr uint32_t N = CB_N, Q2 = 2 * CB_N;
     static_assert(LOGB == PBS_LOGB || (LUT && LIMBS == 2), "the 2^10 gadget: exact LUT-mode form only");
-    KeyPrefetch<S::KEY, 32, 1> next;
+    KeyPrefetch<S::KEY, 32, 1, 512> next;
     const uint32_t pairs = (batch + 1) / 2;
     for (uint32_t pidx = blockIdx.x; pidx < pairs; pidx += gridDim.x) {
         // an odd batch's last workgroup runs its ciphertext twice and stores it once
@@ -657,7 +658,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_split(const uint32_t* __restric
     cplx* own = regions[wv];
     cplx* group = regions[4 * g];
     constexpr uint32_t N = CB_N, Q2 = 2 * CB_N;
-    KeyPrefetch<S::KEY, 16, 2> next;
+    KeyPrefetch<S::KEY, 16, 2, 512> next;
     for (uint32_t cidx = blockIdx.x; cidx < batch; cidx += gridDim.x) {
         __syncthreads();
         const uint32_t bt = pbs_rotations<LUT>(lwe + (size_t)cidx * (n + 1), n, at, io);
