@@ -87,11 +87,11 @@ struct DeviceTables {
 };
 
 // Twiddle tables of the 4-wave N = 2048 FFT (fft1024.hpp): p1t, p2, p3 [4][64],
-// tr [4][4][64], rot [2N]; 5888 complex values.
+// tr [4][4][64], rot [2N], pw [10][16]; 6048 complex values.
 struct DeviceTables1024 {
     FFT1024Tables T{};
     cplx* d_buf = nullptr;
-    static constexpr int kCount = 1792 + 4096;
+    static constexpr int kCount = 1792 + 4096 + 160;
     // host values of the tables, in device order
     static std::vector<cplx> host_values() {
         std::vector<cplx> h(kCount);
@@ -112,6 +112,18 @@ struct DeviceTables1024 {
                     put(768 + (r * 4 + s) * 64 + l, PI * r / N - 2.0 * PI * (double)((r * k) % 1024) / 1024.0);
                 }
         for (int j = 0; j < 2 * N; ++j) put(1792 + j, PI * j / N);
+        for (int L = 0; L < 16; ++L) {
+            const int k = (L >> 2) + 4 * (L & 3);
+            auto pw = [&](int t, int p, int power) {  // (w^4 W256^(k + 16 p))^power, in units of pi / 512
+                put(1792 + 2 * N + t * 16 + L, PI * (double)(((1 - 4 * (k + 16 * p)) * power) % 1024) / 512.0);
+            };
+            pw(0, 0, 4);
+            pw(1, 0, 8);
+            for (int p = 0; p < 4; ++p) {
+                pw(2 + 2 * p, p, 1);
+                pw(3 + 2 * p, p, 2);
+            }
+        }
         return h;
     }
     int init() {
@@ -125,6 +137,7 @@ struct DeviceTables1024 {
         T.p3 = d_buf + 512;
         T.tr = d_buf + 768;
         T.rot = d_buf + 1792;
+        T.pw = d_buf + 1792 + 4096;
         return TFHE_OK;
     }
     void release() {
@@ -150,6 +163,7 @@ struct DeviceTables1024F {
         T.p3 = d_buf + 512;
         T.tr = d_buf + 768;
         T.rot = d_buf + 1792;
+        T.pw = d_buf + 1792 + 4096;
         return TFHE_OK;
     }
     void release() {

@@ -28,6 +28,8 @@ struct FFT1024TablesT {
     const C* tr;   // [4 r][4 s][64 lane]  w^r W1024^(r k(lane, s))
     const C* rot;  // [2N] w^j: frequency k (wave q, slot s, lane) is the polynomial at w^(1 - 4k),
                    // k = (lane >> 4) + 4 ((lane >> 2) & 3) + 16 (lane & 3) + 64 s + 256 q
+    const C* pw;   // [10][16 L = 4 k0 + e] of fft_rows.hpp's fused form: with v = w^4 W256^(k0 + 4 e):
+                   // v^4, v^8, then v_p, v_p^2 for v_p = v W16^p, p < 4
 };
 using FFT1024Tables = FFT1024TablesT<cplx>;
 using FFT1024TablesF = FFT1024TablesT<cplxf>;

@@ -17,6 +17,15 @@
 // k + 256 q.  Reading each value once (4 accesses per lane and transform instead of 16,
 // when every wave read all four inputs for its own quarter of the outputs) also computes
 // each radix-4 once (16 additions instead of 32 FMAs per lane).
+//
+// The exact form's products are rounded to the same integers whatever the order of the FP64
+// operations, so its transforms (suffix _pw) fuse the twiddles into the butterflies: a
+// radix-4 step whose inputs carry w^0 .. w^3 takes 24 FMAs where three twiddle products and the
+// butterfly take 28 operations, and with the twiddles of all steps written as powers (the twist and
+// the previous step's factors together) a lane reads 10 per transform instead of 19.  10% fewer
+// FP64 operations and 7% fewer LDS accesses per step: exact PBS of 128 inputs 6.63 -> 6.45 ms; at full
+// load the clock gives part of it back (1024 inputs 23.3 -> 22.7 ms a round with the HomTrace keys).
+// The one-product form's words depend on every rounding, so it keeps the form above.
 #pragma once
 #include "fft1024.hpp"
 
@@ -33,6 +42,7 @@ struct RowTables {
     const cplx* p3;
 };
 constexpr int ROW_TABLES_CPLX = 256 + 64 + 16;
+constexpr int PW_TABLES_CPLX = 160;  // pw as FFT1024Tables
 
 __device__ __forceinline__ RowTables stage_row_tables(const FFT1024Tables& Tg, cplx* tl) {
     for (int k = threadIdx.x; k < 256; k += blockDim.x) tl[k] = Tg.p1t[k];
@@ -112,6 +122,78 @@ __device__ __forceinline__ void fft256_fwd_rows(cplx (&x)[4][4], cplx* region, c
     }
 }
 
+// x + w y and 2 x - s
+__device__ __forceinline__ cplx cfma(cplx x, cplx w, cplx y) {
+    return {fma(-w.im, y.im, fma(w.re, y.re, x.re)), fma(w.im, y.re, fma(w.re, y.im, x.im))};
+}
+__device__ __forceinline__ cplx twice_less(cplx x, cplx s) { return {fma(2.0, x.re, -s.re), fma(2.0, x.im, -s.im)}; }
+// radix-4 of x[j] w^j, w1 = w, w2 = w^2
+template <bool INV>
+__device__ __forceinline__ void dft4_pw(cplx (&x)[4], cplx w1, cplx w2) {
+    const cplx e = cfma(x[0], w2, x[2]), f = twice_less(x[0], e);
+    const cplx g = cfma(x[1], w2, x[3]), h = twice_less(x[1], g);
+    x[0] = cfma(e, w1, g);
+    x[2] = twice_less(e, x[0]);
+    x[1] = cfma(f, mul_mi<INV>(w1), h);
+    x[3] = twice_less(f, x[1]);
+}
+__device__ __forceinline__ cplx cconj(cplx a) { return {a.re, -a.im}; }
+
+// exp(i pi j / 32) for the constants of the first two steps
+__device__ __forceinline__ cplx pw_const(int j) {
+    constexpr double C[17] = {1.0, 0.99518472667219693, 0.98078528040323043, 0.95694033573220882, 0.92387953251128674,
+                              0.88192126434835505, 0.83146961230254524, 0.77301045336273699, 0.70710678118654757,
+                              0.63439328416364549, 0.55557023301960229, 0.47139673682599764, 0.38268343236508978,
+                              0.29028467725446233, 0.19509032201612828, 0.098017140329560604, 0.0};
+    const int a = j < 0 ? -j : j, im = a <= 16 ? 16 - a : a - 16;  // |j| <= 32
+    const double c = a <= 16 ? C[a] : -C[32 - a], s = C[im];
+    return {c, j < 0 ? -s : s};
+}
+
+// fft256_fwd_rows with the twiddles fused: point b = 64 a + 16 c + d carries v0^b, v0 = w^4, and
+// k = k0 + 4 e + 16 p + 64 s.  Over a: powers of v0^64 = exp(i pi / 8).  Over c: of (v0 W256^k0)^16 =
+// exp(i pi (1 - 4 k0) / 32).  What is left for d is v^d, v = v0 W256^(k0 + 4 e), one v per lane after
+// the transpose (d = 4 g + h): over g powers of v^4, over h powers of v W16^p.  T: pw in LDS.
+template <bool SYNC>
+__device__ __forceinline__ void fft256_fwd_rows_pw(cplx (&x)[4][4], cplx* region, const cplx* T, int lane) {
+    const int R = lane >> 4, d = lane & 15;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        cplx y[4] = {x[0][c], x[1][c], x[2][c], x[3][c]};
+        dft4_pw<false>(y, pw_const(4), pw_const(8));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k][c] = y[k];
+    }
+    if constexpr (SYNC) lds_barrier();
+    cplx* wr = region + R * ROWS_STRIDE + d;
+#pragma unroll
+    for (int k0 = 0; k0 < 4; ++k0) {
+        dft4_pw<false>(x[k0], pw_const(1 - 4 * k0), pw_const(2 - 8 * k0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) wr[(4 * k0 + e) * 17] = x[k0][e];
+    }
+    wave_sync();
+    const int L = d;  // now 4 k0 + e
+    const cplx* rd = region + R * ROWS_STRIDE + L * 17;
+    const cplx t4 = T[L], t8 = T[16 + L];
+    cplx z[4][4];  // [p][h]
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        cplx y[4] = {rd[h], rd[4 + h], rd[8 + h], rd[12 + h]};
+        dft4_pw<false>(y, t4, t8);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) z[p][h] = y[p];
+    }
+    wave_sync();
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        dft4_pw<false>(z[p], T[(2 + 2 * p) * 16 + L], T[(3 + 2 * p) * 16 + L]);
+        cplx* o = region + R * 256 + row_pos(L, p);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) o[s * 64] = z[p][s];
+    }
+}
+
 // Inverse of the same: the region holds [R][s][row_pos(4 k0 + e, p)]; x[a][c] at lane
 // 16 R + d returns 256 x the folded point 64 a + 16 c + d of transform R.
 __device__ __forceinline__ void fft256_inv_rows(cplx (&x)[4][4], cplx* region, const RowTables& T, int lane) {
@@ -123,26 +205,24 @@ __device__ __forceinline__ void fft256_inv_rows(cplx (&x)[4][4], cplx* region, c
         cplx y[4] = {o[0], o[64], o[128], o[192]};
         dft4<true>(y);
 #pragma unroll
-        for (int h = 0; h < 4; ++h) z[h][p] = (h && p) ? cmulc(y[h], w16_const(h * p)) : y[h];
+        for (int h = 0; h < 4; ++h) z[h][p] = y[h];
     }
     wave_sync();
     cplx* wr = region + R * ROWS_STRIDE + L * 17;
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
-        dft4<true>(z[h]);
+        if (h) dft4_pw<true>(z[h], pw_const(4 * h), pw_const(8 * h));  // powers of conj W16^h
+        else dft4<true>(z[h]);
 #pragma unroll
         for (int g = 0; g < 4; ++g) wr[4 * g + h] = z[h][g];
     }
     wave_sync();
     const cplx* rd = region + R * ROWS_STRIDE + d;
-    cplx p2[3];
-#pragma unroll
-    for (int e = 1; e < 4; ++e) p2[e - 1] = T.p2[e * 16 + d];
+    const cplx w1 = cconj(T.p2[16 + d]), w2 = cconj(T.p2[32 + d]);
 #pragma unroll
     for (int k0 = 0; k0 < 4; ++k0) {
-        cplx y[4] = {rd[(4 * k0) * 17], cmulc(rd[(4 * k0 + 1) * 17], p2[0]), cmulc(rd[(4 * k0 + 2) * 17], p2[1]),
-                     cmulc(rd[(4 * k0 + 3) * 17], p2[2])};
-        dft4<true>(y);
+        cplx y[4] = {rd[(4 * k0) * 17], rd[(4 * k0 + 1) * 17], rd[(4 * k0 + 2) * 17], rd[(4 * k0 + 3) * 17]};
+        dft4_pw<true>(y, w1, w2);
 #pragma unroll
         for (int c = 0; c < 4; ++c) x[k0][c] = cmulc(y[c], T.p1t[k0 * 64 + 16 * c + d]);
     }
@@ -159,7 +239,8 @@ __device__ __forceinline__ void fft256_inv_rows(cplx (&x)[4][4], cplx* region, c
 // NT inverse 256-point transforms with 4 points per lane (the layout of fft256_inv) side by
 // side: the twiddle reads are shared and their LDS round trips overlap.  Slot s of lane
 // 16 k0 + 4 e + p in, point 64 a + lane out; region: NT x F256_LDS_CPLX of transposes.
-template <int NT>
+// PW: twiddles fused (the exact form).
+template <int NT, bool PW>
 __device__ __forceinline__ void fft256_inv_multi(cplx (&x)[NT][4], cplx* region, const RowTables& T, int lane) {
     const int k0 = lane >> 4, e = (lane >> 2) & 3, low = lane & 3, d = lane & 15;
 #pragma unroll
@@ -179,9 +260,13 @@ __device__ __forceinline__ void fft256_inv_multi(cplx (&x)[NT][4], cplx* region,
     wave_sync();
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
+        if constexpr (PW) {
+            dft4_pw<true>(x[t], cconj(tw[0]), cconj(tw[1]));
+        } else {
 #pragma unroll
-        for (int p = 1; p < 4; ++p) x[t][p] = cmulc(x[t][p], tw[p - 1]);
-        dft4<true>(x[t]);
+            for (int p = 1; p < 4; ++p) x[t][p] = cmulc(x[t][p], tw[p - 1]);
+            dft4<true>(x[t]);
+        }
 #pragma unroll
         for (int g = 0; g < 4; ++g) region[t * F256_LDS_CPLX + f256_a2(k0, e, 4 * g + low)] = x[t][g];
     }
@@ -195,9 +280,13 @@ __device__ __forceinline__ void fft256_inv_multi(cplx (&x)[NT][4], cplx* region,
     wave_sync();
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
+        if constexpr (PW) {
+            dft4_pw<true>(x[t], cconj(tw[0]), cconj(tw[1]));
+        } else {
 #pragma unroll
-        for (int ee = 1; ee < 4; ++ee) x[t][ee] = cmulc(x[t][ee], tw[ee - 1]);
-        dft4<true>(x[t]);
+            for (int ee = 1; ee < 4; ++ee) x[t][ee] = cmulc(x[t][ee], tw[ee - 1]);
+            dft4<true>(x[t]);
+        }
         row_transpose4(x[t]);
     }
     cplx p1[4];
@@ -220,13 +309,20 @@ __device__ __forceinline__ void load_cross(const FFT1024Tables& Tg, int w, int l
 }
 
 // transform R of the four waves' regions (group: the first wave's region) at this lane's k:
-// slot q = frequency k + 256 q
+// slot q = frequency k + 256 q; PW: T_r = T_1^r fused
+template <bool PW>
 __device__ __forceinline__ void cross_fwd(const cplx* group, int R, int w, int lane, const cplx (&tr)[3], cplx (&x)[4]) {
     const cplx* p = group + R * 256 + w * 64 + row_pos_lane(lane);
-    x[0] = p[0];
+    if constexpr (PW) {
 #pragma unroll
-    for (int r = 1; r < 4; ++r) x[r] = cmul(p[r * ROWS_CPLX], tr[r - 1]);
-    dft4<false>(x);
+        for (int r = 0; r < 4; ++r) x[r] = p[r * ROWS_CPLX];
+        dft4_pw<false>(x, tr[0], tr[1]);
+    } else {
+        x[0] = p[0];
+#pragma unroll
+        for (int r = 1; r < 4; ++r) x[r] = cmul(p[r * ROWS_CPLX], tr[r - 1]);
+        dft4<false>(x);
+    }
 }
 
 // the inverse radix-4 over q and the conjugate cross twiddles; x[r] belongs to wave r

@@ -138,7 +138,7 @@ __device__ __forceinline__ void pbs_mac_rows(cplx (&acc)[2][LIMBS][4], const cpl
     cplx x[4];
 #pragma unroll
     for (int t = 0; t < S::BATCHES; ++t) {
-        if (t % S::BPR == 0) cross_fwd(group, t / S::BPR, w, lane, tr, x);
+        if (t % S::BPR == 0) cross_fwd<LIMBS == 2>(group, t / S::BPR, w, lane, tr, x);
         if (t & 1) S::mac(acc, x, fp, kb, t, fresh);
         else S::mac(acc, x, fp, ka, t, fresh);
         __builtin_amdgcn_sched_barrier(0);
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(256, 2) void k_pbs2(const uint32_t* __restrict__ lw
 #pragma unroll
                 for (int s = 0; s < 4; ++s) y[o][s] = own[o * 256 + s * 64 + lane];
             wave_sync();
-            fft256_inv_multi<2>(y, own, T, lane);
+            fft256_inv_multi<2, false>(y, own, T, lane);
 #pragma unroll
             for (int o = 0; o < 2; ++o)
 #pragma unroll
@@ -439,6 +439,9 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict
     __shared__ cplx regions[8][ROWS_CPLX];
     __shared__ cplx tl[ROW_TABLES_CPLX];
     __shared__ uint16_t at[2][1024];
+    __shared__ cplx tpw[LIMBS == 2 ? PW_TABLES_CPLX : 1];
+    if constexpr (LIMBS == 2)
+        for (int k = threadIdx.x; k < PW_TABLES_CPLX; k += blockDim.x) tpw[k] = Tg.pw[k];
     const RowTables T = stage_row_tables(Tg, tl);
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -508,8 +511,13 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict
                     digit_rows<LOGB>(acc[u], x);
                     // u = 1: the other waves read this wave's region until the barrier; u = 0:
                     // only this wave has used it since the inverse transform's exchange
-                    if (u == 0) fft256_fwd_rows<false>(x, own, T, lane);
-                    else fft256_fwd_rows<true>(x, own, T, lane);
+                    if constexpr (LIMBS == 2) {
+                        if (u == 0) fft256_fwd_rows_pw<false>(x, own, tpw, lane);
+                        else fft256_fwd_rows_pw<true>(x, own, tpw, lane);
+                    } else {
+                        if (u == 0) fft256_fwd_rows<false>(x, own, T, lane);
+                        else fft256_fwd_rows<true>(x, own, T, lane);
+                    }
                 }
                 cplx kv[P::DEPTH][4];
 #pragma unroll
@@ -528,10 +536,17 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict
 #pragma unroll
                         for (int c = 0; c < 2; ++c) {
                             const cplx* p = &regions[4 * (c ^ cc)][rd + (t / S::BPR) * 256];
-                            const cplx a = cadd(p[0], cmul(p[2 * ROWS_CPLX], trf[1]));
-                            const cplx b = cadd(cmul(p[ROWS_CPLX], trf[0]), cmul(p[3 * ROWS_CPLX], trf[2]));
-                            x[c][0] = cadd(a, b);
-                            x[c][1] = csub(a, b);
+                            if constexpr (LIMBS == 2) {  // T_3 = T_1 T_2
+                                const cplx a = cfma(p[0], trf[1], p[2 * ROWS_CPLX]);
+                                const cplx b = cfma(p[ROWS_CPLX], trf[1], p[3 * ROWS_CPLX]);
+                                x[c][0] = cfma(a, trf[0], b);
+                                x[c][1] = twice_less(a, x[c][0]);
+                            } else {
+                                const cplx a = cadd(p[0], cmul(p[2 * ROWS_CPLX], trf[1]));
+                                const cplx b = cadd(cmul(p[ROWS_CPLX], trf[0]), cmul(p[3 * ROWS_CPLX], trf[2]));
+                                x[c][0] = cadd(a, b);
+                                x[c][1] = csub(a, b);
+                            }
                         }
                     }
                     pr.mac(x, kv[t % P::DEPTH], u, t);
@@ -597,7 +612,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict
 #pragma unroll
                     for (int s = 0; s < 4; ++s) y[o][s] = own[512 + o * 256 + s * 64 + lane];
                 wave_sync();
-                fft256_inv_multi<2>(y, own, T, lane);
+                fft256_inv_multi<2, false>(y, own, T, lane);
 #pragma unroll
                 for (int o = 0; o < 2; ++o)
 #pragma unroll
@@ -645,6 +660,9 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_split(const uint32_t* __restric
     __shared__ cplx regions[8][ROWS_CPLX];
     __shared__ cplx tl[ROW_TABLES_CPLX];
     __shared__ uint16_t at[1024];
+    __shared__ cplx tpw[LIMBS == 2 ? PW_TABLES_CPLX : 1];
+    if constexpr (LIMBS == 2)
+        for (int k = threadIdx.x; k < PW_TABLES_CPLX; k += blockDim.x) tpw[k] = Tg.pw[k];
     const RowTables T = stage_row_tables(Tg, tl);
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -683,7 +701,8 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_split(const uint32_t* __restric
             {
                 cplx x[4][4];
                 digit_rows<LOGB>(acc, x);
-                fft256_fwd_rows<false>(x, own, T, lane);
+                if constexpr (LIMBS == 2) fft256_fwd_rows_pw<false>(x, own, tpw, lane);
+                else fft256_fwd_rows<false>(x, own, T, lane);
             }
             S::load(ka, step, kat, g, 0, g, 1 - g);
             S::load(kb, step, kat, g, 1, g, 1 - g);
@@ -723,7 +742,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_split(const uint32_t* __restric
 #pragma unroll
                 for (int s = 0; s < 4; ++s) y[lb][s] = own[512 + lb * 256 + s * 64 + lane];
             wave_sync();
-            fft256_inv_multi<LIMBS>(y, own, T, lane);
+            fft256_inv_multi<LIMBS, LIMBS == 2>(y, own, T, lane);
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
                 if constexpr (LIMBS == 1) {
