@@ -26,7 +26,7 @@ struct DeviceTables {
     cplx* d_buf = nullptr;
     int init(int N) {
         if (N != 1024) return fail(TFHE_E_PARAM, "FFT tables: only N = 1024 is built");
-        std::vector<cplx> h(1024 + 2 * N + 1024 + PAIR_TABLE_CPLX);
+        std::vector<cplx> h(1024 + 2 * N + 1024 + PAIR_TABLE_CPLX + 6 * 64);
         const double PI = 3.14159265358979323846264338327950288;
         for (int k = 0; k < 8; ++k)
             for (int b = 0; b < 64; ++b) {
@@ -69,6 +69,22 @@ struct DeviceTables {
                     put(128 + 32 * p + n + 16 * b8, th / 32 + PI * ((p >> 2) / 16.0 + ((p >> 1) & 1) / 8.0 + (p & 1) / 4.0) +
                                                         PI / 2 * b8);
         }
+        // Pw256Regs at lane 16 k0 + .. (powers over c), 4 (4 k0 + e) + .. (over g), 16 k0 + 4 e + p (over h)
+        cplx* h4 = h3 + 384;
+        for (int l = 0; l < 64; ++l) {
+            const int k0 = l >> 4, k = k0 + 4 * ((l >> 2) & 3), p = l & 3;
+            // exp(i pi / 512 (1 - 4 k) m)
+            auto put = [&](int idx, int kk, int m) {
+                const double ang = PI * (double)(((1 - 4 * kk) * m) % 1024) / 512.0;
+                h4[idx * 64 + l] = {std::cos(ang), std::sin(ang)};
+            };
+            put(0, k0, 16);
+            put(1, k0, 32);
+            put(2, k, 4);
+            put(3, k, 8);
+            put(4, k + 16 * p, 1);
+            put(5, k + 16 * p, 2);
+        }
         int rc = dmalloc((void**)&d_buf, h.size() * sizeof(cplx));
         if (rc) return rc;
         rc = hipcheck(hipMemcpy(d_buf, h.data(), h.size() * sizeof(cplx), hipMemcpyHostToDevice), "tables");
@@ -78,6 +94,7 @@ struct DeviceTables {
         T.rot = d_buf + 1024;
         T.two = d_buf + 1024 + 2 * N;
         T.pair = T.two + 1024;
+        T.pw = T.pair + 384;
         return TFHE_OK;
     }
     void release() {

@@ -191,6 +191,7 @@ struct FFTTables {
     const cplx* p2;   // [8][64]
     const cplx* rot;  // [2N] w^j, w = exp(i pi / N): X[k] of the transform is p(w^(1 - 4k))
     const cplx* pair;  // twiddles of fft512_pair.hpp
+    const cplx* pw;   // two-wave transform with fused twiddles: Pw256Regs [6][64]
     const cplx* two;  // two-wave transform: p1t, p2, p3 [4][64] of fft1024.hpp, cross twiddles [256]
 };
 

@@ -55,6 +55,34 @@ __device__ __forceinline__ void dft4(C (&x)[4]) {
     x[3] = csub(a1, b1);
 }
 
+// x + w y and 2 x - s
+__device__ __forceinline__ cplx cfma(cplx x, cplx w, cplx y) {
+    return {fma(-w.im, y.im, fma(w.re, y.re, x.re)), fma(w.im, y.re, fma(w.re, y.im, x.im))};
+}
+__device__ __forceinline__ cplx twice_less(cplx x, cplx s) { return {fma(2.0, x.re, -s.re), fma(2.0, x.im, -s.im)}; }
+// radix-4 of x[j] w^j, w1 = w, w2 = w^2
+template <bool INV>
+__device__ __forceinline__ void dft4_pw(cplx (&x)[4], cplx w1, cplx w2) {
+    const cplx e = cfma(x[0], w2, x[2]), f = twice_less(x[0], e);
+    const cplx g = cfma(x[1], w2, x[3]), h = twice_less(x[1], g);
+    x[0] = cfma(e, w1, g);
+    x[2] = twice_less(e, x[0]);
+    x[1] = cfma(f, mul_mi<INV>(w1), h);
+    x[3] = twice_less(f, x[1]);
+}
+__device__ __forceinline__ cplx cconj(cplx a) { return {a.re, -a.im}; }
+
+// exp(i pi j / 32) for the constants of the first two steps
+__device__ __forceinline__ cplx pw_const(int j) {
+    constexpr double C[17] = {1.0, 0.99518472667219693, 0.98078528040323043, 0.95694033573220882, 0.92387953251128674,
+                              0.88192126434835505, 0.83146961230254524, 0.77301045336273699, 0.70710678118654757,
+                              0.63439328416364549, 0.55557023301960229, 0.47139673682599764, 0.38268343236508978,
+                              0.29028467725446233, 0.19509032201612828, 0.098017140329560604, 0.0};
+    const int a = j < 0 ? -j : j, im = a <= 16 ? 16 - a : a - 16;  // |j| <= 32
+    const double c = a <= 16 ? C[a] : -C[32 - a], s = C[im];
+    return {c, j < 0 ? -s : s};
+}
+
 __device__ __forceinline__ int f256_a1(int k0, int b) { return k0 * 80 + (b >> 4) * 20 + (b & 15); }
 
 // The first transpose of the forward 256-point step (and the last of the inverse, its own
@@ -175,6 +203,63 @@ __device__ __forceinline__ void fft256_inv(C (&x)[4], C* lds, const Tw& T, int l
     dft4<true>(x);
 #pragma unroll
     for (int a = 1; a < 4; ++a) x[a] = cmulc(x[a], twist4_const<C>(a));
+}
+
+// The 256-point step with the twiddles fused into the butterflies (for products that are rounded
+// to integers, whose words do not depend on the order of the FP64 operations): point
+// b = 64 a + 16 c + d carries v0^b, v0 = w^4, and k = k0 + 4 e + 16 p + 64 s; over c powers of
+// (v0 W256^k0)^16, over g and h (d = 4 g + h) powers of v^4 and v W16^p, v = v0 W256^(k0 + 4 e).
+struct Pw256Regs {  // each pair: the factor and its square at this lane
+    cplx w[6];
+    __device__ __forceinline__ Pw256Regs(const cplx* t, int lane) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) w[k] = t[k * 64 + lane];
+    }
+};
+__device__ __forceinline__ void fft256_fwd_pw(cplx (&x)[4], cplx* lds, const Pw256Regs& T, int lane) {
+    dft4_pw<false>(x, pw_const(4), pw_const(8));
+    row_transpose4(x);
+    const int k0 = lane >> 4, d = lane & 15, e = (lane >> 2) & 3, low = lane & 3;
+    dft4_pw<false>(x, T.w[0], T.w[1]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) lds[f256_a2(k0, q, d)] = x[q];
+    wave_sync();
+#pragma unroll
+    for (int g = 0; g < 4; ++g) x[g] = lds[f256_a2(k0, e, 4 * g + low)];
+    wave_sync();
+    dft4_pw<false>(x, T.w[2], T.w[3]);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) lds[f256_a3(k0, e, p, low)] = x[p];
+    wave_sync();
+#pragma unroll
+    for (int h = 0; h < 4; ++h) x[h] = lds[f256_a3(k0, e, low, h)];
+    wave_sync();
+    dft4_pw<false>(x, T.w[4], T.w[5]);
+}
+template <class Tw>
+__device__ __forceinline__ void fft256_inv_pw(cplx (&x)[4], cplx* lds, const Tw& T, int lane) {
+    dft4<true>(x);
+    const int k0 = lane >> 4, e = (lane >> 2) & 3, low = lane & 3, d = lane & 15;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) lds[f256_a3(k0, e, low, h)] = x[h];
+    wave_sync();
+#pragma unroll
+    for (int p = 0; p < 4; ++p) x[p] = lds[f256_a3(k0, e, p, low)];
+    wave_sync();
+    dft4_pw<true>(x, cconj(T.p3(1)), cconj(T.p3(2)));
+#pragma unroll
+    for (int g = 0; g < 4; ++g) lds[f256_a2(k0, e, 4 * g + low)] = x[g];
+    wave_sync();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x[q] = lds[f256_a2(k0, q, d)];
+    wave_sync();
+    dft4_pw<true>(x, cconj(T.p2(1)), cconj(T.p2(2)));
+    row_transpose4(x);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k] = cmulc(x[k], T.p1(k));
+    dft4<true>(x);
+#pragma unroll
+    for (int a = 1; a < 4; ++a) x[a] = cmulc(x[a], twist4_const<cplx>(a));
 }
 
 // Cross-wave step of the FFT1024 (wave w holds frequencies 256 w ..): forward and

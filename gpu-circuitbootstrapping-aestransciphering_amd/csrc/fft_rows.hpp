@@ -122,34 +122,6 @@ __device__ __forceinline__ void fft256_fwd_rows(cplx (&x)[4][4], cplx* region, c
     }
 }
 
-// x + w y and 2 x - s
-__device__ __forceinline__ cplx cfma(cplx x, cplx w, cplx y) {
-    return {fma(-w.im, y.im, fma(w.re, y.re, x.re)), fma(w.im, y.re, fma(w.re, y.im, x.im))};
-}
-__device__ __forceinline__ cplx twice_less(cplx x, cplx s) { return {fma(2.0, x.re, -s.re), fma(2.0, x.im, -s.im)}; }
-// radix-4 of x[j] w^j, w1 = w, w2 = w^2
-template <bool INV>
-__device__ __forceinline__ void dft4_pw(cplx (&x)[4], cplx w1, cplx w2) {
-    const cplx e = cfma(x[0], w2, x[2]), f = twice_less(x[0], e);
-    const cplx g = cfma(x[1], w2, x[3]), h = twice_less(x[1], g);
-    x[0] = cfma(e, w1, g);
-    x[2] = twice_less(e, x[0]);
-    x[1] = cfma(f, mul_mi<INV>(w1), h);
-    x[3] = twice_less(f, x[1]);
-}
-__device__ __forceinline__ cplx cconj(cplx a) { return {a.re, -a.im}; }
-
-// exp(i pi j / 32) for the constants of the first two steps
-__device__ __forceinline__ cplx pw_const(int j) {
-    constexpr double C[17] = {1.0, 0.99518472667219693, 0.98078528040323043, 0.95694033573220882, 0.92387953251128674,
-                              0.88192126434835505, 0.83146961230254524, 0.77301045336273699, 0.70710678118654757,
-                              0.63439328416364549, 0.55557023301960229, 0.47139673682599764, 0.38268343236508978,
-                              0.29028467725446233, 0.19509032201612828, 0.098017140329560604, 0.0};
-    const int a = j < 0 ? -j : j, im = a <= 16 ? 16 - a : a - 16;  // |j| <= 32
-    const double c = a <= 16 ? C[a] : -C[32 - a], s = C[im];
-    return {c, j < 0 ? -s : s};
-}
-
 // fft256_fwd_rows with the twiddles fused: point b = 64 a + 16 c + d carries v0^b, v0 = w^4, and
 // k = k0 + 4 e + 16 p + 64 s.  Over a: powers of v0^64 = exp(i pi / 8).  Over c: of (v0 W256^k0)^16 =
 // exp(i pi (1 - 4 k0) / 32).  What is left for d is v^d, v = v0 W256^(k0 + 4 e), one v per lane after

@@ -349,7 +349,8 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
     __shared__ uint16_t at[1024];
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const Tw256Regs T({Tg.two, Tg.two + 256, Tg.two + 512, nullptr, nullptr}, lane);
+    const Tw256Regs T({Tg.two, Tg.two + 256, Tg.two + 512, nullptr, nullptr, nullptr}, lane);
+    const Pw256Regs F(Tg.pw, lane);
     constexpr uint32_t q = 2u * N;
     constexpr uint32_t OFF = digit_offset32<GATE_LOGB, GATE_L>();
     const int r = w & 1, row = w >> 1, j = row >> 1, u = row & 1;  // forward role
@@ -417,7 +418,7 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
             for (int a = 0; a < 4; ++a)
                 x[a] = {(double)((int32_t)(((vr[a] + OFF) >> sh) & BM) - HB),
                         (double)((int32_t)(((vi[a] + OFF) >> sh) & BM) - HB)};
-            fft256_fwd(x, bufs[w], T, lane);
+            fft256_fwd_pw(x, bufs[w], F, lane);
 #pragma unroll
             for (int s = 0; s < 4; ++s) bufs[w][s * 64 + lpos] = x[s];
         };
@@ -438,17 +439,18 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
             __syncthreads();
             for (int i = 0; i < n; ++i) {
                 const uint32_t mrot = (q - uniform(at[i])) & (q - 1);
+                // w^(m (1 - 4k)); read here, where nothing waits for the gather's bank conflicts
+                const cplx z = rot[(mrot * ek) & (q - 1u)];
                 forward();
                 lds_barrier();
                 cplx s0 = {0.0, 0.0}, s1 = {0.0, 0.0};
 #pragma unroll
                 for (int t = 0; t < GATE_ROWS; ++t) {
-                    const cplx y0 = bufs[2 * t][pos], y1 = cmul(bufs[2 * t + 1][pos], cross);
-                    cmac(s0, cadd(y0, y1), kv[t][0]);
-                    cmac(s1, csub(y0, y1), kv[t][1]);
+                    const cplx y0 = bufs[2 * t][pos], z0 = cfma(y0, cross, bufs[2 * t + 1][pos]);
+                    cmac(s0, z0, kv[t][0]);
+                    cmac(s1, twice_less(y0, z0), kv[t][1]);
                 }
                 // times w^(m (1 - 4k)) - 1 (exactly 0 for m = 0); w^(m (1 - 4(k + 256))) is (-1)^m of it
-                const cplx z = rot[(mrot * ek) & (q - 1u)];
                 const double sg = (mrot & 1) ? -1.0 : 1.0;
                 s0 = cmul(s0, {z.re - 1.0, z.im});
                 s1 = cmul(s1, {fma(sg, z.re, -1.0), sg * z.im});
@@ -468,7 +470,7 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
                 cplx x[4];
 #pragma unroll
                 for (int s = 0; s < 4; ++s) x[s] = prod[iv][r][s * 64 + lpos];
-                fft256_inv(x, bufs[w], T, lane);
+                fft256_inv_pw(x, bufs[w], T, lane);
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
                     acc[a] += round_mod32(x[a].re, 1.0 / M);
