@@ -351,6 +351,7 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Tw256Regs T({Tg.two, Tg.two + 256, Tg.two + 512, nullptr, nullptr, nullptr}, lane);
     const Pw256Regs F(Tg.pw, lane);
+    const double magic = round_magic();
     constexpr uint32_t q = 2u * N;
     constexpr uint32_t OFF = digit_offset32<GATE_LOGB, GATE_L>();
     const int r = w & 1, row = w >> 1, j = row >> 1, u = row & 1;  // forward role
@@ -401,23 +402,29 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
                 acc[s] = iv ? gate_tv(q1, q2, bt, c, q) : 0u;
             }
         }
+        // published ready for the digits: the offset added, the top bit of each digit flipped (as the
+        // batched form keeps its accumulator), so that a digit is one signed bit field
+        uint32_t flip = 0;
+#pragma unroll
+        for (int l = 0; l < GATE_L; ++l) flip |= 1u << (32 - GATE_L * GATE_LOGB + (l + 1) * GATE_LOGB - 1);
         auto publish = [&]() {
+            uint32_t v[8];
+#pragma unroll
+            for (int h = 0; h < 8; ++h) v[h] = (acc[h] + OFF) ^ flip;
 #pragma unroll
             for (int h = 0; h < 2; ++h)
-                accw[iv][r][h][lane] = make_uint4(acc[4 * h], acc[4 * h + 1], acc[4 * h + 2], acc[4 * h + 3]);
+                accw[iv][r][h][lane] = make_uint4(v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]);
         };
         // the transform of this wave's half digit row
         auto forward = [&]() {
             const uint4 re = accw[u][r][0][lane], im = accw[u][r][1][lane];
             const uint32_t vr[4] = {re.x, re.y, re.z, re.w}, vi[4] = {im.x, im.y, im.z, im.w};
             const int sh = 32 - GATE_L * GATE_LOGB + j * GATE_LOGB;
-            constexpr uint32_t BM = (1u << GATE_LOGB) - 1;
-            constexpr int HB = 1 << (GATE_LOGB - 1);
             cplx x[4];
 #pragma unroll
             for (int a = 0; a < 4; ++a)
-                x[a] = {(double)((int32_t)(((vr[a] + OFF) >> sh) & BM) - HB),
-                        (double)((int32_t)(((vi[a] + OFF) >> sh) & BM) - HB)};
+                x[a] = {(double)(int32_t)__builtin_amdgcn_sbfe(vr[a], (uint32_t)sh, GATE_LOGB),
+                        (double)(int32_t)__builtin_amdgcn_sbfe(vi[a], (uint32_t)sh, GATE_LOGB)};
             fft256_fwd_pw(x, bufs[w], F, lane);
 #pragma unroll
             for (int s = 0; s < 4; ++s) bufs[w][s * 64 + lpos] = x[s];
@@ -473,8 +480,8 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
                 fft256_inv_pw(x, bufs[w], T, lane);
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
-                    acc[a] += round_mod32(x[a].re, 1.0 / M);
-                    acc[a + 4] += round_mod32(x[a].im, 1.0 / M);
+                    acc[a] += round_mod32(x[a].re, 1.0 / M, magic);
+                    acc[a + 4] += round_mod32(x[a].im, 1.0 / M, magic);
                 }
                 publish();
                 lds_barrier();
