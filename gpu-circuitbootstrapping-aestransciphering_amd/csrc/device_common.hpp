@@ -257,6 +257,28 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Barrier over some of a workgroup's waves: each adds one to a counter in LDS (zero at the kernel's
+// start) and reads it until it holds `target`, the number of arrivals so far of all those waves.
+// Every one of them passes the same barriers and a workgroup's waves are all resident, so the wait
+// ends.  LDS accesses of a wave are performed in order: its writes before the barrier are seen by
+// whoever sees its arrival.
+__device__ __forceinline__ void wave_group_barrier(uint32_t* counter, uint32_t target) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)counter;
+    uint32_t one = 1, seen;
+    uint64_t lanes;
+    asm volatile(
+        "s_mov_b64 %1, exec\n s_mov_b64 exec, 1\n"
+        "ds_add_u32 %2, %3\n"
+        "1: ds_read_b32 %0, %2\n s_waitcnt lgkmcnt(0)\n"
+        "v_readfirstlane_b32 vcc_lo, %0\n s_cmp_lt_u32 vcc_lo, %4\n s_cbranch_scc1 1b\n"
+        "s_mov_b64 exec, %1\n"
+        : "=&v"(seen), "=&s"(lanes)
+        : "v"(at), "v"(one), "s"(target)
+        : "vcc", "scc", "memory");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // forward: x = folded coefficient pairs (untwisted), out in frequency distribution
 __device__ __forceinline__ void fft512_fwd(cplx (&x)[8], cplx* lds, const FFTTables& T, int lane) {
 #pragma unroll
