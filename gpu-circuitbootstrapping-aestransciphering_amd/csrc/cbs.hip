@@ -1448,9 +1448,10 @@ void launch_gen_pfkl40(uint64_t seed, const int32_t* K2, int8_t* KT, hipStream_t
 
 void launch_pfkl(const uint64_t* lwe64, uint32_t B, int8_t* D, const int8_t* KT, int u0, int nu, uint32_t* out,
                  size_t out_stride, size_t out_u_offset, hipStream_t st) {
-    // many input tiles: the LDS-staged form (256-input tiles, one 8-wave workgroup per CU);
-    // few: 128-input tiles, for twice the workgroups
-    const bool staged = B > 1792;
+    // more than one 256-input tile: the LDS-staged form (one 8-wave workgroup per CU; 320 inputs
+    // 0.27 ms against 0.37 in 128-input tiles, 512 0.30 / 0.40, 768 0.50 / 0.57, 1024 0.57 / 0.74); one:
+    // 128-input tiles, for twice the workgroups
+    const bool staged = B > 256;
     const uint32_t Mpad = staged ? (B + 255) / 256 * 256 : (B + 127) / 128 * 128;
     k_pfkl_digits<<<grid_for((size_t)Mpad * (PFKL_KP / 8) / 256 + 1, 8192), 256, 0, st>>>(lwe64, B, Mpad, D);
     const unsigned rows = Mpad / 128, tiles = (unsigned)nu * 2 * CB_N / 64;
