@@ -243,6 +243,11 @@ __device__ __forceinline__ cplx key_at(const cplx* base, uint32_t at) {
     const v2d v = *(__attribute__((address_space(1))) const v2d*)(b + at);
     return {v.x, v.y};
 }
+// entry k, uniform over the wave, of a table that no kernel writes: a scalar load
+__device__ __forceinline__ cplx uniform_at(const cplx* base, uint32_t k) {
+    auto p = (__attribute__((address_space(4))) const double*)base + 2 * k;
+    return {p[0], p[1]};
+}
 // a lane's 32-bit offset as a value of the block it is used in (once per batch of loads): one
 // widened outside the loop would hide that it fits 32 bits
 __device__ __forceinline__ uint32_t fresh_offset(uint32_t at) {
@@ -349,6 +354,12 @@ __device__ __forceinline__ double round_magic() {
 __device__ __forceinline__ uint32_t round_mod32(double x, double scale, double magic = ROUND_MAGIC) {
     const double y = fma(x, scale, magic);
     return (uint32_t)__double_as_longlong(y);
+}
+
+// the same of a value that carries its scale already: one addition (the fused form needs a copy of
+// the constant for every value)
+__device__ __forceinline__ uint32_t round_add_mod32(double x, double magic) {
+    return (uint32_t)__double_as_longlong(x + magic);
 }
 
 // Signed digits by the offset method: with off = 2^(IGN-1) + sum_j (B/2) 2^(IGN + j logB),

@@ -132,7 +132,8 @@ __device__ __forceinline__ uint32_t gate_tv(uint32_t q1, uint32_t q2, uint32_t b
 // FP64 of 3,080 vector instructions per step, two waves per SIMD: 77% of the issue slots at
 // the clock the chip holds under FMA load).  With one radix-8 transform per wave at a time
 // (two LDS round trips each, eight in a row) 1000 / 2048 / 4096 gates took 6.5 / 11.2 / 21.2 ms;
-// now 6.2 / 10.5 / 19.9.  Per step: the digit rows
+// now 6.0 / 10.4 / 19.8 (the monic update's
+// table values are loaded before the last keys, the inverse's 1 / M is in its factors).  Per step: the digit rows
 // of both polynomials by pairs (fft512_pair.hpp), the Fourier-domain MAC against the
 // streamed BSK row block, the two inverse transforms as one pair, exact rounding mod 2^32 and
 // the CGGI monic update acc += X^m t - t with m = -a~_i mod 2N (reference
@@ -219,6 +220,7 @@ __global__ __launch_bounds__(256, 2) void k_gate_blind_rotate(
             if (mrot == 0) continue;
             const cplx* key = bskf + (size_t)(i0 + i) * GATE_ROWS * 2 * M;
             cplx macc[2][8];
+            cplx z0, g1, g2, g3;
 #pragma unroll
             for (int j = 0; j < GATE_L; ++j) {
                 cplx x[16];
@@ -239,6 +241,12 @@ __global__ __launch_bounds__(256, 2) void k_gate_blind_rotate(
                     for (int p = 0; p < 4; ++p)
                         kv[t % KD][p] = key_at(key + (4 * j + t / 2) * M + (4 * (t & 1) + p) * 64, at);
                 };
+                if (j == GATE_L - 1) {  // the monic update's table values, ahead of the last keys
+                    z0 = Tg.rot[(mrot * e0) & (q - 1)];
+                    g1 = uniform_at(Tg.rot, (64u * mrot) & (q - 1));
+                    g2 = uniform_at(Tg.rot, (128u * mrot) & (q - 1));
+                    g3 = uniform_at(Tg.rot, (256u * mrot) & (q - 1));
+                }
 #pragma unroll
                 for (int t = 0; t < KD; ++t) load(t);
                 __builtin_amdgcn_sched_barrier(0);
@@ -262,21 +270,17 @@ __global__ __launch_bounds__(256, 2) void k_gate_blind_rotate(
             // rotating the rounded t.  One table lookup per lane (a gather of one cache line per
             // lane), turned by the powers of w^(64 m) for the p of a lane
             {
-                const cplx z0 = Tg.rot[(mrot * e0) & (q - 1)];
-                const cplx g1 = key_at(Tg.rot, ((64u * mrot) & (q - 1)) * (uint32_t)sizeof(cplx));
-                const cplx g2 = key_at(Tg.rot, ((128u * mrot) & (q - 1)) * (uint32_t)sizeof(cplx));
-                const cplx g3 = key_at(Tg.rot, ((256u * mrot) & (q - 1)) * (uint32_t)sizeof(cplx));
                 cplx z[8];  // p = 4 b5 + 2 b6 + b7: exponent + 64 b5 + 128 b6 + 256 b7
-                z[0] = z0;
-                z[4] = cmul(z0, g1);
-                z[2] = cmul(z0, g2);
+                z[0] = {z0.re * (1.0 / M), z0.im * (1.0 / M)};  // the inverse's 1 / M
+                z[4] = cmul(z[0], g1);
+                z[2] = cmul(z[0], g2);
                 z[6] = cmul(z[4], g2);
 #pragma unroll
                 for (int p = 0; p < 8; p += 2) z[p + 1] = cmul(z[p], g3);
 #pragma unroll
                 for (int o = 0; o < 2; ++o)
 #pragma unroll
-                    for (int p = 0; p < 8; ++p) macc[o][p] = cmul(macc[o][p], {z[p].re - 1.0, z[p].im});
+                    for (int p = 0; p < 8; ++p) macc[o][p] = cmul(macc[o][p], {z[p].re - 1.0 / M, z[p].im});
             }
             // output o to half o
             cplx x[16];
@@ -289,8 +293,8 @@ __global__ __launch_bounds__(256, 2) void k_gate_blind_rotate(
             fft512_pair_inv(x, A, tab, lane);
 #pragma unroll
             for (int a = 0; a < 16; ++a) {
-                re[a] += round_mod32(x[a].re, 1.0 / M, magic);
-                im[a] += round_mod32(x[a].im, 1.0 / M, magic);
+                re[a] += round_add_mod32(x[a].re, magic);
+                im[a] += round_add_mod32(x[a].im, magic);
             }
         }
     }
