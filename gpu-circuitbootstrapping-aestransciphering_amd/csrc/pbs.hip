@@ -368,6 +368,9 @@ __global__ __launch_bounds__(256, 2) void k_pbs2(const uint32_t* __restrict__ lw
 // with hp = wv >> 2, of BOTH ciphertexts, so that one key load feeds two products: the key
 // stream (196 KB per wave and step in the two-bit form when each ciphertext loads its own) is
 // what a step waits on most at this size of launch.
+// A wave runs its products and inverse transforms at a higher priority than its forward ones: left
+// to the SIMD's order by age, the older of its two waves ran a whole forward transform ahead of the
+// younger one's inverse, which then ran alone (17 blocks 283.5 -> 280.4 ms; exact, 8 blocks, 352.9 -> 350.0).
 template <int LIMBS, int MB, bool ANYM>
 struct PbsPair {
     using S = PbsStep<LIMBS, MB, ANYM>;
@@ -500,6 +503,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict
             if ((m1[0] | m1[1] | m2[0] | m2[1]) == 0) continue;
             const cplx* step = bskf + (size_t)(i / MB) * S::KEY;
             P pr;
+            __builtin_amdgcn_s_setprio(0);
             if constexpr (MB == 2 && !LUT) {
 #pragma unroll
                 for (int c = 0; c < 2; ++c) pr.factors(Tg.rot, c, m1[c], m2[c], ek);
@@ -527,6 +531,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict
 #pragma unroll
                     for (int c = 0; c < 2; ++c) pr.factors(Tg.rot, c, fresh_uniform(m1[c]), fresh_uniform(m2[c]), ek);
                 }
+                __builtin_amdgcn_s_setprio(2);
                 lds_barrier();
                 const int rd = w * 64 + row_pos_lane(lane);
                 cplx x[2][2];
@@ -554,6 +559,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_pair(const uint32_t* __restrict
                     if (t + P::DEPTH < S::BATCHES) P::load(kv[t % P::DEPTH], step, kat, u, t + P::DEPTH);
                     __builtin_amdgcn_sched_barrier(0);
                 }
+                if (u == 0) __builtin_amdgcn_s_setprio(0);
             }
             next.touch(i + MB < n ? step + S::KEY : step);
             if constexpr (MB == 1) {
@@ -690,6 +696,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_split(const uint32_t* __restric
     constexpr uint32_t N = CB_N, Q2 = 2 * CB_N;
     KeyPrefetch<S::KEY, 16, 2, 512> next;
     uint32_t arrivals = 0;
+    if (g) __builtin_amdgcn_s_setprio(1);  // one group ahead of the other (1 block fast 34.0 -> 33.4 ms, exact 77.8 -> 77.1)
     for (uint32_t cidx = first; cidx < batch; cidx += stride) {
         __syncthreads();
         const uint32_t bt = pbs_rotations<LUT>(lwe + (size_t)cidx * (n + 1), n, at, io);
