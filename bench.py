@@ -750,7 +750,7 @@ def aes_headline(args):
         traffic = json.load(open(prof)).get("hbm_bytes_per_launch")
     head = {"value": round(blocks * args.steps / elapsed, 3), "elapsed_s": elapsed, "blocks_wrong": bad,
             "keygen_s": round(keygen_s, 2), "tuned_shapes": tuned,
-            "roofline": {"bound": "valu", "kernel": "k_pbs2_manylut (" + form_text(approx, mb, lin, l2r, ksl)[0] + ")",
+            "roofline": {"bound": "valu", "kernel": "k_pbs2_pair (" + form_text(approx, mb, lin, l2r, ksl)[0] + ")",
                          "achieved": round(tflops, 3), "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                          "frac": round(tflops / PEAK_FP64_TFLOPS, 4),
                          "traffic": traffic if args.aes_form in ("approx-auto-lin", "approx-auto-links") else None,

@@ -132,7 +132,7 @@ __device__ __forceinline__ uint32_t gate_tv(uint32_t q1, uint32_t q2, uint32_t b
 // FP64 of 3,080 vector instructions per step, two waves per SIMD: 77% of the issue slots at
 // the clock the chip holds under FMA load).  With one radix-8 transform per wave at a time
 // (two LDS round trips each, eight in a row) 1000 / 2048 / 4096 gates took 6.5 / 11.2 / 21.2 ms;
-// now 6.0 / 10.4 / 19.8 (the monic update's
+// now 6.0 / 10.3 / 19.8 (the monic update's
 // table values are loaded before the last keys, the inverse's 1 / M is in its factors).  Per step: the digit rows
 // of both polynomials by pairs (fft512_pair.hpp), the Fourier-domain MAC against the
 // streamed BSK row block, the two inverse transforms as one pair, exact rounding mod 2^32 and

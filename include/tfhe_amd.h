@@ -413,10 +413,10 @@ int tfhe_cbs_keyswitch_batch(tfhe_cbs_ctx* ctx, const uint32_t* d_lwe32, uint32_
 /* Launch-shape autotuner (no counterpart in the reference, whose shapes are fixed at
  * compile time): times, with events on `stream`, the candidate shapes of one AES
  * round over `blocks` blocks and keeps the fastest in the context for later calls
- * of those sizes.  choices[5] receives the PBS form (0 branchy, 1 branch-free FFT step;
- * with two key bits per step 1 = the wide key batch at one wave per SIMD, 0 = two
- * waves per SIMD, 2 = split over 8 waves; in a pbs_multibit = 3 context 0 / 1 are one
- * bit per step and 2 / 3 / 4 two bits at two waves per SIMD / wide / split) of the
+ * of those sizes.  choices[5] receives the PBS form (exact: 0 = two ciphertexts per
+ * workgroup, 1 = one split over 8 waves; one-product, one bit per step: one form; two key
+ * bits per step: 0 / 1 = two ciphertexts per workgroup, 2 = split; in a pbs_multibit = 3
+ * context 0 / 1 are one bit per step and 2 / 3 / 4 those of two bits) of the
  * full-round part and of the rest of tfhe_cbs_batch's split,
  * the PFKS i-slices of the same two parts, and the N=2048 key switch's i-slices;
  * -1 where a part does not exist.  A part of 16 or more rounds of resident

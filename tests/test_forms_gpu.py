@@ -141,3 +141,48 @@ def test_pbs_pairs_and_odd_batches(gpu, okeys, form):
     if form in ("exact", "htss"):
         assert np.array_equal(d_one.cpu().numpy(), rows[257][:3])
     c.close()
+
+
+@pytest.mark.parametrize("params", [{}, {"pbs_approx": 1, "pbs_multibit": 2}], ids=["exact", "two_bits"])
+def test_pbs_small_launches(gpu, okeys, params):
+    """Up to 64 inputs run 16 to an XCD, more are dealt to all of them: a prefix of a launch of 128
+    gives its rows, and nothing past it is written."""
+    import torch
+    import tfhe_amd
+    c = tfhe_amd.CbsContext(max_blocks=1, params=tfhe_amd.cbs_params(**params))
+    c.keygen(okeys.s, SEED)
+    d_cts = to_dev(_rand((128, okeys.p.n + 1), 4))
+    d_all = torch.empty((128, 2, 2049), dtype=torch.int64, device="cuda")
+    c.pbs_batch(d_cts, d_all)
+    for count in (1, 15, 17, 33, 50, 64, 65):
+        d_out = torch.full((count + 1, 2, 2049), 7, dtype=torch.int64, device="cuda")
+        c.pbs_batch(d_cts[:count].contiguous(), d_out[:count])
+        torch.cuda.synchronize()
+        assert torch.equal(d_out[:count], d_all[:count]), count
+        assert bool((d_out[count] == 7).all())
+    c.close()
+
+
+def test_pfks_linear_counts(gpu, okeys):
+    """Linear PFKS: 128-input tiles up to 256 inputs, 256-input tiles staged through LDS above; the
+    rows of each launch equal those of launches of 64, and the oracle's on the first and last."""
+    import torch
+    import tfhe_amd
+    c = tfhe_amd.CbsContext(max_blocks=3, params=tfhe_amd.cbs_params(pfks_linear=1))
+    c.keygen(okeys.s, SEED)
+    lwe = _rand((600, 2049), 6, 64)
+    d_in = torch.from_numpy(lwe.view(np.int64).copy()).to("cuda")
+    for u in (0, 1):
+        d_ref = torch.empty((600, 4096), dtype=torch.int32, device="cuda")
+        for k in range(0, 600, 64):
+            m = min(64, 600 - k)
+            c.pfks_batch(u, d_in[k:k + m].contiguous(), m, 4096, d_ref[k:k + m])
+        for count in (1, 128, 255, 256, 257, 511, 513, 600):
+            d_out = torch.full((count + 1, 4096), 7, dtype=torch.int32, device="cuda")
+            c.pfks_batch(u, d_in[:count].contiguous(), count, 4096, d_out)
+            torch.cuda.synchronize()
+            assert torch.equal(d_out[:count], d_ref[:count]), (u, count)
+            assert bool((d_out[count] == 7).all())
+        for k in (0, 599):
+            assert np.array_equal(from_dev(d_ref)[k], okeys.pfks_linear(u, lwe[k])), (u, k)
+    c.close()
