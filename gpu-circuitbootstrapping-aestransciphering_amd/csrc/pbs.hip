@@ -820,6 +820,7 @@ int pbs_model_form(uint32_t batch, int limbs, int mb) {
 template <bool LUT>
 static void launch_pbs2_t(const uint32_t* lwe, uint32_t batch, int n, const cplx* bskf, int limbs, int mb,
                           const FFT1024Tables& T, uint64_t* out, hipStream_t st, int form, const PbsLut& io) {
+    if (!batch) return;
     const unsigned grid = batch < 2048 ? batch : 2048;  // one workgroup per ciphertext (or pair) at a time
     const unsigned pairs = (batch + 1) / 2, pgrid = pairs < 2048 ? pairs : 2048;
     // The split form of up to 64 ciphertexts runs on as many XCDs as give each 16: the workgroups of
