@@ -509,7 +509,20 @@ __global__ __launch_bounds__(64 * GSPLIT_WAVES, 1) void k_gate_blind_rotate_spli
 // per blind-rotation step a decompose+FFT launch (one wavefront per digit row),
 // a MAC+inverse-FFT launch (one wavefront per output polynomial) and a monic
 // update launch, for one ciphertext at a time.
+// A step waits on its launches' chains of loads.  Digit transforms and products are in the key's
+// frequency order, so that its values are read 64 consecutive ones at a time, and the products
+// run on 8 waves, one position per thread and all of its 12 loads in flight; the sums come back to
+// the transform's order through LDS.  One gate 5.81 ms; 6.83 with one wave that gathered the
+// key's values at the transform's frequencies, 6.52 with a key in the transform's own order.
 // ===========================================================================
+// the key's position of this lane's frequency f of fft512_fwd
+__device__ __forceinline__ uint32_t plain_freq(int lane, int f) {
+    return pair_pos((uint32_t)((lane >> 3) + 8 * (lane & 7) + 64 * f));
+}
+// place in LDS of position p: adjacent lanes differ in p's bits 0, 7 and 8 in the transform's
+// order and in bits 0..2 in the key's, and both touch all banks
+__device__ __forceinline__ uint32_t plain_pos(uint32_t p) { return p ^ ((p >> 6) & 2u) ^ ((p >> 6) & 4u); }
+
 __global__ __launch_bounds__(64) void k_plain_decompose_fft(const uint32_t* __restrict__ acc, FFTTables T,
                                                            cplx* __restrict__ digf) {
     __shared__ cplx lds[FFT512_LDS_CPLX];
@@ -526,24 +539,30 @@ __global__ __launch_bounds__(64) void k_plain_decompose_fft(const uint32_t* __re
     }
     fft512_fwd(x, lds, T, lane);
 #pragma unroll
-    for (int f = 0; f < 8; ++f) digf[(r * 8 + f) * 64 + lane] = x[f];
+    for (int f = 0; f < 8; ++f) digf[r * 512 + plain_freq(lane, f)] = x[f];
 }
 
-__global__ __launch_bounds__(64) void k_plain_mac_ifft(const cplx* __restrict__ digf, const cplx* __restrict__ key,
+__global__ __launch_bounds__(512) void k_plain_mac_ifft(const cplx* __restrict__ digf, const cplx* __restrict__ key,
                                                       FFTTables T, uint32_t* __restrict__ t) {
     __shared__ cplx lds[FFT512_LDS_CPLX];
-    const int lane = threadIdx.x, o = blockIdx.x;
-    cplx x[8];
-    uint32_t kpos[8];  // the key's positions of this lane's frequencies
+    const int p = threadIdx.x, o = blockIdx.x;
+    cplx d[GATE_ROWS], k[GATE_ROWS];
 #pragma unroll
-    for (int f = 0; f < 8; ++f) {
-        x[f] = {0.0, 0.0};
-        kpos[f] = pair_pos((uint32_t)((lane >> 3) + 8 * (lane & 7) + 64 * f));
+    for (int r = 0; r < GATE_ROWS; ++r) {
+        d[r] = digf[r * 512 + p];
+        k[r] = key[(r * 2 + o) * 512 + p];
     }
-    for (int r = 0; r < GATE_ROWS; ++r)
+    cplx sum = {0.0, 0.0};
 #pragma unroll
-        for (int f = 0; f < 8; ++f)
-            cmac(x[f], digf[(r * 8 + f) * 64 + lane], key[(r * 2 + o) * 512 + kpos[f]]);
+    for (int r = 0; r < GATE_ROWS; ++r) cmac(sum, d[r], k[r]);
+    lds[plain_pos((uint32_t)p)] = sum;
+    __syncthreads();
+    if (p >= 64) return;
+    const int lane = p;
+    cplx x[8];
+#pragma unroll
+    for (int f = 0; f < 8; ++f) x[f] = lds[plain_pos(plain_freq(lane, f))];
+    wave_sync();
     fft512_inv(x, lds, T, lane);
 #pragma unroll
     for (int a = 0; a < 8; ++a) {
@@ -831,7 +850,7 @@ void launch_plain_init(uint32_t* acc, uint32_t q1, uint32_t bt, hipStream_t st) 
 void launch_plain_step(uint32_t* acc, cplx* digf, uint32_t* t, const cplx* key, uint32_t m,
                        const FFTTables& T, hipStream_t st) {
     k_plain_decompose_fft<<<GATE_ROWS, 64, 0, st>>>(acc, T, digf);
-    k_plain_mac_ifft<<<2, 64, 0, st>>>(digf, key, T, t);
+    k_plain_mac_ifft<<<2, 512, 0, st>>>(digf, key, T, t);
     k_plain_monic<<<2, 256, 0, st>>>(acc, t, m);
 }
 
@@ -847,7 +866,7 @@ void launch_polymul1024(const int32_t* x, const uint32_t* y, uint32_t batch, con
 void launch_external_product1024(uint32_t* acc, cplx* digf, uint32_t* t, const cplx* key, const FFTTables& T,
                                  hipStream_t st) {
     k_plain_decompose_fft<<<GATE_ROWS, 64, 0, st>>>(acc, T, digf);
-    k_plain_mac_ifft<<<2, 64, 0, st>>>(digf, key, T, t);
+    k_plain_mac_ifft<<<2, 512, 0, st>>>(digf, key, T, t);
 }
 
 uint32_t ks_bpad(uint32_t batch) { return (batch + KS_GROUP - 1) / KS_GROUP * KS_GROUP; }
