@@ -1420,6 +1420,14 @@ uint32_t pfks_bpad(uint32_t B) { return (B + PF_PAD - 1) / PF_PAD * PF_PAD; }
 // per load), more take 512 inputs x 128 columns, so that the key is read once for all of them
 // (512 inputs: 3.40 ms against 3.49 in two groups of 256; 320: 2.79 against 3.4)
 static int pfks_halves(uint32_t B) { return B <= 256 ? 2 : 1; }
+// The last inputs of a launch that would fill at most half of a workgroup's 512 run as a launch of
+// their own, in the other shape: a workgroup's time is its fullest wave's, so they would cost what
+// 512 do (one function, ms: 513 inputs 2.50 against 3.37 in one launch, 768 2.86 / 3.55, 1280 4.49 / 5.12;
+// both functions 514 4.9 / 5.7, 768 5.3 / 6.3)
+static uint32_t pfks_rest(uint32_t B) {
+    const uint32_t rest = B % 512;
+    return B > 512 && rest <= 256 ? rest : 0;
+}
 
 void launch_pfks_digits(const uint64_t* lwe64, uint32_t B, uint32_t* at, hipStream_t st) {
     const uint32_t Bpad = pfks_bpad(B);
@@ -1442,6 +1450,7 @@ void launch_zero_rows32(uint32_t* out, uint32_t count, size_t stride, uint32_t w
 }
 
 int pfks_model_slices(uint32_t B, int nu) {
+    B -= pfks_rest(B);
     // i-slices (4..32): the launch runs in rounds of as many workgroups as fit at once
     // (one of 16 waves per CU), and a workgroup's time is its slice
     // length, so pick the slice count with the fewest rounds x coefficients per
@@ -1464,13 +1473,18 @@ int pfks_model_slices(uint32_t B, int nu) {
 
 void launch_pfks32(const uint32_t* at, uint32_t B, const uint32_t* key, size_t key_u_stride, int u0, int nu,
                    uint32_t* out, size_t out_stride, size_t out_u_offset, hipStream_t st, int slices) {
-    if (slices <= 0) slices = pfks_model_slices(B, nu);
-    if (slices > CB_N + 1) slices = CB_N + 1;
-    const unsigned h = (unsigned)pfks_halves(B), per_group = PF_WAVES / h * PF_CT;
-    dim3 grid(2 * CB_N / (128 * h), (B + per_group - 1) / per_group, (unsigned)(slices * nu));
-    auto kernel = h == 2 ? k_pfks32<2> : k_pfks32<1>;
-    kernel<<<grid, 64 * PF_WAVES, 0, st>>>(at, B, pfks_bpad(B), key, key_u_stride, u0, slices, out, out_stride,
-                                            out_u_offset);
+    const uint32_t Bpad = pfks_bpad(B), rest = pfks_rest(B);
+    auto launch = [&](uint32_t first, uint32_t count, int sl) {
+        if (sl <= 0) sl = pfks_model_slices(count, nu);
+        if (sl > CB_N + 1) sl = CB_N + 1;
+        const unsigned h = (unsigned)pfks_halves(count), per_group = PF_WAVES / h * PF_CT;
+        dim3 grid(2 * CB_N / (128 * h), (count + per_group - 1) / per_group, (unsigned)(sl * nu));
+        auto kernel = h == 2 ? k_pfks32<2> : k_pfks32<1>;
+        kernel<<<grid, 64 * PF_WAVES, 0, st>>>(at + first, count, Bpad, key, key_u_stride, u0, sl,
+                                                out + (size_t)first * out_stride, out_stride, out_u_offset);
+    };
+    launch(0, B - rest, slices);
+    if (rest) launch(B - rest, rest, 0);
 }
 
 size_t pfkl_key_bytes() { return (size_t)2 * PFKL_SLICES * 2 * CB_N * PFKL_KP; }

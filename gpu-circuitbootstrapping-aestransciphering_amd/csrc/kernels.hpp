@@ -121,7 +121,8 @@ int launch_ks_linear(const uint32_t* lwe32, uint32_t count, int n, const int8_t*
 // LWEs as a u64 mask array (rows a_stride apart) and a u64 body array -> [batch][n+1] u32
 void launch_pack_lwe64(const uint64_t* a, const uint64_t* b, uint32_t batch, int n, uint32_t a_stride, uint32_t* out,
                        hipStream_t st);
-// slices <= 0: the resident-workgroup cost model (pfks_model_slices); > 0: that many i-slices
+// slices <= 0: the resident-workgroup cost model (pfks_model_slices); > 0: that many i-slices (of the
+// whole groups of 512 inputs; a rest of at most 256 after them is a launch with the model's own)
 int pfks_model_slices(uint32_t B, int nu);
 void launch_pfks32(const uint32_t* at, uint32_t B, const uint32_t* key, size_t key_u_stride, int u0, int nu,
                    uint32_t* out, size_t out_stride, size_t out_u_offset, hipStream_t st, int slices = 0);

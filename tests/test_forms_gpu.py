@@ -186,3 +186,63 @@ def test_pfks_linear_counts(gpu, okeys):
         for k in (0, 599):
             assert np.array_equal(from_dev(d_ref)[k], okeys.pfks_linear(u, lwe[k])), (u, k)
     c.close()
+
+
+@pytest.mark.parametrize("count", [640, 767, 768, 769, 1025, 1280, 1281])
+def test_pfks_rest_launch(ctx, okeys, count):
+    """Lookup PFKS of whole groups of 512 inputs and a rest: up to 256 of it run as a launch of their
+    own, more in the groups' launch; each row equals the oracle's, at a stride wider than a row."""
+    import torch
+    base = _rand((5, 2049), 15, 64)
+    pick = np.arange(count) * 3 % 5
+    d_in = torch.from_numpy(base[pick].view(np.int64).copy()).to("cuda")
+    for u in (0, 1):
+        d_out = torch.full((count + 1, 4100), 7, dtype=torch.int32, device="cuda")
+        ctx.pfks_batch(u, d_in, count, 4100, d_out)
+        torch.cuda.synchronize()
+        got = from_dev(d_out)
+        want = np.stack([okeys.pfks(u, base[j]) for j in range(5)])
+        assert np.array_equal(got[:count, :4096], want[pick]), u
+        assert (got[count] == 7).all() and (got[:, 4096:] == 7).all()
+
+
+@pytest.mark.parametrize("count", [257, 320, 384, 385, 600])
+def test_cbs_rest_launch(ctx, okeys, count):
+    """The same with both functions in a launch (2 count PFKS inputs of a circuit bootstrap batch):
+    the rows of batches of 64."""
+    import torch
+    d_in = to_dev(_rand((count, okeys.p.n + 1), 16))
+    d_out = torch.full((count + 1, 4, 2, 2048), 7, dtype=torch.int32, device="cuda")
+    ctx.cbs_batch(d_in, d_out[:count])
+    d_ref = torch.empty((count, 4, 2, 2048), dtype=torch.int32, device="cuda")
+    for k in range(0, count, 64):
+        ctx.cbs_batch(d_in[k:k + 64].contiguous(), d_ref[k:k + 64])
+    torch.cuda.synchronize()
+    assert torch.equal(d_out[:count], d_ref)
+    assert bool((d_out[count] == 7).all())
+
+
+def _least_ms(fn, passes=8):
+    import torch
+    fn()
+    best = float("inf")
+    for _ in range(passes):
+        t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        t0.record()
+        fn()
+        t1.record()
+        torch.cuda.synchronize()
+        best = min(best, t0.elapsed_time(t1))
+    return best
+
+
+def test_pfks_rest_is_not_a_whole_group(ctx):
+    """600 lookup PFKS take no longer than launches of 512 and 88 do (1.35 times as long when the 88
+    waited in a whole group's time); 1.15 allows for what two timings differ by."""
+    import torch
+    d_in = torch.from_numpy(_rand((600, 2049), 17, 64).view(np.int64).copy()).to("cuda")
+    d_out = torch.empty((600, 4096), dtype=torch.int32, device="cuda")
+    whole = _least_ms(lambda: ctx.pfks_batch(1, d_in, 600, 4096, d_out))
+    parts = (_least_ms(lambda: ctx.pfks_batch(1, d_in, 512, 4096, d_out)) +
+             _least_ms(lambda: ctx.pfks_batch(1, d_in[512:], 88, 4096, d_out[512:])))
+    assert whole < 1.15 * parts, (whole, parts)
