@@ -811,26 +811,26 @@ typedef int pfkl_v16i __attribute__((ext_vector_type(16)));
 // v_mfma_i32_32x32x32_i8: lane l holds 16 bytes of A row (l % 32) and of B column
 // (l % 32) at k = 16 (l / 32) + 0..15; accumulator register j of lane l is
 // C[8 (j / 4) + 4 (l / 32) + j % 4][l % 32].
-// Grid x = Mpad / 128 input tiles, y = nu * 2N / 64 column tiles.  Wave w computes
+// Grid x = nu * 2N / 64 column tiles, y = Mpad / 128 input tiles.  Wave w computes
 // 64 inputs (m0 + 0..63, two 32-row blocks) x 32 columns x 5 slices: ten 16-register
 // accumulators (160 registers, held in AGPRs), one 16-byte digit load per row block and
 // one key load per slice per 32 k.  One wave per SIMD leaves the registers for four
 // operand sets in flight: the loads are latency-bound, and two steps of prefetch beat
-// two waves per SIMD with one (3.34 against 3.78 ms per 17-block round).  The pairs of
+// two waves per SIMD with one (3.34 against 3.78 ms at 4352 inputs of both functions, a size that
+// the staged form serves now).  The pairs of
 // waves that read the same digit or key fragment are kept within four steps of each
 // other by a workgroup barrier, so that the second read of a fragment finds it in L1
-// (8192 inputs: 6.13 -> 5.96 ms per function pair, same words).
+// (6.13 -> 5.96 ms at 8192 inputs, same words).
 __global__ __launch_bounds__(256, 1) void k_pfkl_gemm(const int8_t* __restrict__ D, uint32_t B,
                                                   const int8_t* __restrict__ KT, int u0,
                                                   uint32_t* __restrict__ out, size_t out_stride,
-                                                  size_t out_u_offset, int cols_first) {
+                                                  size_t out_u_offset) {
     constexpr int COLS = 2 * CB_N;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // cols_first: blockIdx.x = column tile, blockIdx.y = row block, so that the row blocks of one
-    // key tile have linear workgroup ids 128 apart, on one XCD (a launch of at most two row
-    // blocks runs whole, and the second read of each key tile hits that XCD's L2)
-    const uint32_t rb = cols_first ? blockIdx.y : blockIdx.x, ct = cols_first ? blockIdx.x : blockIdx.y;
+    // the input tiles of one key tile have linear workgroup ids 64 or 128 apart, on one XCD: all
+    // run at once (launch_pfkl), and the further reads of a key tile hit that XCD's L2
+    const uint32_t rb = blockIdx.y, ct = blockIdx.x;
     const uint32_t m0 = rb * 128 + (w & 1) * 64;
     const uint32_t cg = ct * 64 + (w >> 1) * 32;
     const int uu = (int)(cg / COLS), col0 = (int)(cg % COLS);
@@ -1500,19 +1500,19 @@ void launch_gen_pfkl40(uint64_t seed, const int32_t* K2, int8_t* KT, hipStream_t
 
 void launch_pfkl(const uint64_t* lwe64, uint32_t B, int8_t* D, const int8_t* KT, int u0, int nu, uint32_t* out,
                  size_t out_stride, size_t out_u_offset, hipStream_t st) {
-    // more than one 256-input tile: the LDS-staged form (one 8-wave workgroup per CU; 320 inputs
-    // 0.27 ms against 0.37 in 128-input tiles, 512 0.30 / 0.40, 768 0.50 / 0.57, 1024 0.57 / 0.74); one:
-    // 128-input tiles, for twice the workgroups
-    const bool staged = B > 256;
+    // 128-input tiles while one round of workgroups holds them all (256 inputs of both functions, 512 of
+    // one), above that 256-input tiles staged through LDS, one 8-wave workgroup per CU.  Staged against
+    // 128-input tiles, ms: both functions 320 inputs 0.27 / 0.37, 512 0.30 / 0.40, 768 0.50 / 0.57, 1024
+    // 0.57 / 0.74; one function 300 inputs 0.25 / 0.20 (half the CUs get a staged workgroup), 600 0.27 / 0.38,
+    // 1000 0.31 / 0.40
+    const bool staged = (B + 127) / 128 * nu * (2 * CB_N / 64) > device_cus();
     const uint32_t Mpad = staged ? (B + 255) / 256 * 256 : (B + 127) / 128 * 128;
     k_pfkl_digits<<<grid_for((size_t)Mpad * (PFKL_KP / 8) / 256 + 1, 8192), 256, 0, st>>>(lwe64, B, Mpad, D);
-    const unsigned rows = Mpad / 128, tiles = (unsigned)nu * 2 * CB_N / 64;
+    const unsigned tiles = (unsigned)nu * 2 * CB_N / 64;
     if (staged)
         k_pfkl_gemm_lds<<<dim3(Mpad / 256, tiles), 512, 0, st>>>(D, B, KT, u0, out, out_stride, out_u_offset);
-    else if (rows <= 2)
-        k_pfkl_gemm<<<dim3(tiles, rows), 256, 0, st>>>(D, B, KT, u0, out, out_stride, out_u_offset, 1);
     else
-        k_pfkl_gemm<<<dim3(rows, tiles), 256, 0, st>>>(D, B, KT, u0, out, out_stride, out_u_offset, 0);
+        k_pfkl_gemm<<<dim3(tiles, Mpad / 128), 256, 0, st>>>(D, B, KT, u0, out, out_stride, out_u_offset);
 }
 
 size_t kskl_key_bytes() { return (size_t)KSL_SLICES * KSL_COLS * PFKL_KP; }

@@ -246,3 +246,31 @@ def test_pfks_rest_is_not_a_whole_group(ctx):
     parts = (_least_ms(lambda: ctx.pfks_batch(1, d_in, 512, 4096, d_out)) +
              _least_ms(lambda: ctx.pfks_batch(1, d_in[512:], 88, 4096, d_out[512:])))
     assert whole < 1.15 * parts, (whole, parts)
+
+
+def test_pfks_linear_one_function(gpu, okeys):
+    """Linear PFKS of one function: 128-input tiles up to 512 inputs, where one round of workgroups
+    holds them.  The rows of 385, 512 and 513 inputs are those of launches of 64, and 300
+    inputs take about what 256 do (1.27 times as long in staged 256-input tiles, which leave half of
+    the chip idle there; 1.15 allows for what two timings differ by)."""
+    import torch
+    import tfhe_amd
+    c = tfhe_amd.CbsContext(max_blocks=3, params=tfhe_amd.cbs_params(pfks_linear=1))
+    c.keygen(okeys.s, SEED)
+    d_in = torch.from_numpy(_rand((513, 2049), 18, 64).view(np.int64).copy()).to("cuda")
+    d_out = torch.full((514, 4096), 7, dtype=torch.int32, device="cuda")
+    for u in (0, 1):
+        d_ref = torch.empty((513, 4096), dtype=torch.int32, device="cuda")
+        for k in range(0, 513, 64):
+            m = min(64, 513 - k)
+            c.pfks_batch(u, d_in[k:k + m].contiguous(), m, 4096, d_ref[k:k + m])
+        for count in (385, 512, 513):
+            d_out.fill_(7)
+            c.pfks_batch(u, d_in, count, 4096, d_out)
+            torch.cuda.synchronize()
+            assert torch.equal(d_out[:count], d_ref[:count]), (u, count)
+            assert bool((d_out[count] == 7).all())
+    t256 = _least_ms(lambda: c.pfks_batch(1, d_in, 256, 4096, d_out), 20)
+    t300 = _least_ms(lambda: c.pfks_batch(1, d_in, 300, 4096, d_out), 20)
+    assert t300 < 1.15 * t256, (t300, t256)
+    c.close()
