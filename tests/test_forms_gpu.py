@@ -274,3 +274,111 @@ def test_pfks_linear_one_function(gpu, okeys):
     t300 = _least_ms(lambda: c.pfks_batch(1, d_in, 300, 4096, d_out), 20)
     assert t300 < 1.15 * t256, (t300, t256)
     c.close()
+
+
+def _phase64(K2, r):
+    return O.rlwe_phase64(K2, np.ascontiguousarray(r).reshape(-1)).astype(np.uint64)
+
+
+@pytest.mark.parametrize("form", ["exact", "one_bit", "two_bits", "htss"])
+def test_many_lut_forms(gpu, okeys, form):
+    """A caller's test polynomial in the launches that two ciphertexts share (257 and 258 inputs) and in
+    small ones, at bitwidths 0 and 1: rotations are odd and even at 0, so the factors of a
+    lane's frequencies differ, and even at 1.  Inputs: random words, a zero mask, one rotating key
+    bit.  Exact forms: the oracle's words, of the last odd input too.  One-product forms: every
+    coefficient's phase within 2^40 of 2^64 of the exact oracle's (both carry the PBS noise, about
+    2^36 rms)."""
+    import os
+    from concurrent.futures import ThreadPoolExecutor
+    import torch
+    import tfhe_amd
+    params = {"exact": {}, "one_bit": {"pbs_approx": 1}, "two_bits": {"pbs_approx": 1, "pbs_multibit": 2},
+              "htss": {"lwe_to_rgsw": 1}}[form]
+    keys = O.CbsKeys(SEED, p=O.cbs_params_htss()) if form == "htss" else okeys
+    mb = 2 if form == "two_bits" else 1
+    if mb == 2:
+        keys.bsk_mb2_fourier()
+    c = tfhe_amd.CbsContext(max_blocks=3, params=tfhe_amd.cbs_params(**params))
+    c.keygen(keys.s, SEED)
+    cts = _rand((258, keys.p.n + 1), 19)
+    cts[1, :-1] = 0
+    cts[2, :-1] = 0
+    cts[2, 7] = 0x2345678
+    cts[255] = cts[1]
+    lut = _rand(keys.p.N, 20, 64)
+    d_lut = torch.from_numpy(lut.view(np.int64).copy()).to("cuda")
+    rows = [0, 1, 2, 3, 255, 256, 257]
+    for bw in (0, 1):
+        with ThreadPoolExecutor(max(1, min(16, os.cpu_count() or 1))) as pool:
+            want = dict(zip(rows, pool.map(lambda k: keys.bootstrap_many_lut(cts[k], lut, bw, mb=mb), rows)))
+        for count in (4, 257, 258):
+            d_out = torch.full((count + 1, 2, keys.p.N), 7, dtype=torch.int64, device="cuda")
+            c.bootstrap_many_lut(to_dev(cts[:count]), d_lut, bw, d_out[:count])
+            torch.cuda.synchronize()
+            got = from_dev(d_out, np.uint64)
+            assert (got[count] == 7).all()
+            for k in rows:
+                if k >= count:
+                    continue
+                exact, err = want[k]
+                assert err < 0.25
+                if form in ("exact", "htss") or k in (1, 255):  # a zero mask: no products
+                    assert np.array_equal(got[k], exact), (bw, count, k)
+                else:
+                    d = (_phase64(keys.K2, got[k]) - _phase64(keys.K2, exact)).view(np.int64)
+                    assert np.abs(d).max() < 2 ** 40, (bw, count, k)
+    c.close()
+
+
+@pytest.mark.parametrize("form", ["one_bit", "two_bits"])
+def test_one_product_forms_agree(gpu, okeys, form):
+    """One key bit per step is one kernel at every size: 3 inputs and 257 give the same words.  Two key
+    bits: two ciphertexts per workgroup (form 0) and one split over 8 waves (form 2) sum in
+    another order; a zero mask (no products) gives the same words, and one rotating key bit a phase
+    within 2^30 of 2^64 (the first step's rounding is 2^25 rms).  The last odd input of 257 agrees
+    with the oracle's exact bootstrap within 2^40."""
+    import torch
+    import tfhe_amd
+    mb = 2 if form == "two_bits" else 1
+    c = tfhe_amd.CbsContext(max_blocks=3, params=tfhe_amd.cbs_params(pbs_approx=1, pbs_multibit=mb))
+    c.keygen(okeys.s, SEED)
+    cts = _rand((257, okeys.p.n + 1), 21)
+    cts[:3, :-1] = 0
+    cts[1, 7] = 1 << 29
+    cts[2, 400] = 0x9abcdef0
+
+    def run(count):
+        d_out = torch.full((count + 1, 2, 2049), 7, dtype=torch.int64, device="cuda")
+        c.pbs_batch(to_dev(cts[:count]), d_out[:count])
+        torch.cuda.synchronize()
+        assert bool((d_out[count] == 7).all())
+        return from_dev(d_out, np.uint64)[:count]
+
+    large = run(257)
+    K = okeys.K2.astype(np.int64).astype(np.uint64)
+
+    def apart(a, b):  # phases of two outputs, both levels
+        d = (a[:, -1] - (a[:, :-1] * K).sum(1, dtype=np.uint64)) - (b[:, -1] - (b[:, :-1] * K).sum(1, dtype=np.uint64))
+        return int(np.abs(d.view(np.int64)).max())
+
+    if mb == 1:
+        assert np.array_equal(run(3), large[:3])
+        assert np.array_equal(run(256), large[:256])
+    else:
+        for count in (3, 256):
+            pinned = {}
+            for f in (0, 2):
+                c.set_pbs_form(count, f)
+                pinned[f] = run(count)
+            c.set_pbs_form(count, -1)
+            assert np.array_equal(run(count), pinned[2])  # the size rule's choice
+            assert np.array_equal(pinned[0], large[:count])
+            assert np.array_equal(pinned[2][0], large[0])
+            for k in (1, 2):
+                assert apart(pinned[2][k], large[k]) < 2 ** 30, (count, k)
+            for k in range(3, count):
+                assert apart(pinned[2][k], large[k]) < 2 ** 40, (count, k)
+    want, err = okeys.pbs_mb2(cts[256]) if mb == 2 else okeys.pbs(cts[256])
+    assert err < 0.25
+    assert apart(large[256], want) < 2 ** 40
+    c.close()
