@@ -247,7 +247,7 @@ struct tfhe_cbs_ctx {
     hipStream_t cstream = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     // launch shapes chosen by tfhe_cbs_autotune, keyed by the launch's size (absent: the
-    // kernels' own models): PBS inputs -> FFT form, PFKS LWEs -> i-slices, key switches -> i-slices
+    // kernels' own models): PBS inputs -> form, PFKS LWEs -> i-slices, key switches -> i-slices
     std::map<uint32_t, int> tune_pbs, tune_pfks, tune_ks;
     // kernel timing (tfhe_cbs_timing_enable / _read): an event pair around every PBS launch
     // made outside stream capture while enabled; the pairs are reused after each read
@@ -750,11 +750,10 @@ static int check_cbs(const tfhe_cbs_ctx* c, uint32_t batch, uint32_t cap) {
     return TFHE_OK;
 }
 
-// pbs_multibit = 3 without a tuned choice: two key bits per step at every size (with the key
-// loads batched it measured faster than one bit at 128, 2048 and 8192 inputs: 5.9 / 34.4 /
-// 136 ms against 8.1 / 44.4 / 178), split over 8 waves (4) for launches of at most one
-// workgroup per CU, else at two waves per SIMD (2); 3 is the wide key batch.  Forms 0 and 1
-// are one bit per step with that FFT form.
+// pbs_multibit = 3 without a tuned choice: two key bits per step at every size (ms against one
+// bit's: 100 inputs 3.2 / 5.5, 256 4.0 / 5.6, 512 6.4 / 9.4, 2176 30.0 / 37.1), split over 8 waves (4)
+// for launches of at most one workgroup per CU, else two ciphertexts per workgroup (2; 3 is the
+// same).  Forms 0 and 1 are one bit per step.
 static int auto_pbs_model(uint32_t batch) { return 2 + pbs_model_form(batch, 1, 2); }
 
 // The HomTrace form's PBS: the accumulator (0, LUT X^-b~) with its test polynomial, b + 2^30
@@ -805,7 +804,7 @@ extern "C" int tfhe_cbs_pbs_batch(tfhe_cbs_ctx* c, const uint32_t* d_lwe, uint32
                                   "(tfhe_cbs_bootstrap_many_lut gives them)");
     if (!batch) return TFHE_OK;
     int mb = pbs_mb(c->p), form = tuned(c->tune_pbs, batch, -1);
-    if (pbs_auto(c->p)) {  // forms 2 and 3 = two key bits per step, else one bit with that FFT form
+    if (pbs_auto(c->p)) {  // forms 2 .. 4 = two key bits per step, else one bit
         if (form < 0) form = auto_pbs_model(batch);
         mb = form >= 2 ? 2 : 1;
         if (mb == 2) form -= 2;
@@ -1111,7 +1110,7 @@ int tune_one(hipStream_t st, hipEvent_t e0, hipEvent_t e1, const std::vector<int
 
 // Times the launch shapes of one AES round over `blocks` blocks (128 circuit bootstraps
 // per block) and keeps the fastest in the context for later calls of that size: the PBS
-// FFT form of each part of tfhe_cbs_batch's split, the PFKS i-slices of each part and
+// form of each part of tfhe_cbs_batch's split, the PFKS i-slices of each part and
 // the N=2048 key switch's i-slices.  Inputs are hash-filled context buffers; the round
 // state, RGSW and LUT buffers of the context are overwritten.  The choices change
 // launch shapes only: the exact PBS, the PFKS and the key switch give the same words.
@@ -1185,12 +1184,13 @@ extern "C" int tfhe_cbs_autotune(tfhe_cbs_ctx* c, uint32_t blocks, int* choices,
         const int model_form = pbs_auto(c->p) ? auto_pbs_model(batch) : pbs_model_form(batch, limbs, mb);
         int form = model_form;
         if (model_form >= 0) {
-            // auto contexts: 2 / 3 / 4 = two key bits per step (two waves per SIMD / wide /
-            // split over 8 waves), 0 / 1 = one bit with that FFT form
+            // each kernel once (auto contexts: 4 / 2 = two key bits per step, split over 8 waves / two
+            // ciphertexts per workgroup, 1 = one bit; the other numbers are aliases)
             std::vector<int> cand{model_form};
-            for (int f : pbs_auto(c->p) ? std::vector<int>{4, 3, 2, 1, 0}
-                         : mb == 2        ? std::vector<int>{2, 1, 0}
-                                          : std::vector<int>{1 - model_form})
+            for (int f : pbs_auto(c->p) ? std::vector<int>{4, 2, 1}
+                         : mb == 2        ? std::vector<int>{2, 0}
+                         : limbs == 2     ? std::vector<int>{1, 0}
+                                          : std::vector<int>{1})
                 if (f != model_form) cand.push_back(f);
             const cplx* bsk2 = c->d_bsk2f + bsk2_mb2_first(c->p) * 8 * 2 * 1024;
             rc = tune_one(st, e0, e1, cand, budget_ms,

@@ -414,11 +414,12 @@ int tfhe_cbs_keyswitch_batch(tfhe_cbs_ctx* ctx, const uint32_t* d_lwe32, uint32_
  * compile time): times, with events on `stream`, the candidate shapes of one AES
  * round over `blocks` blocks and keeps the fastest in the context for later calls
  * of those sizes.  choices[5] receives the PBS form (exact: 0 = two ciphertexts per
- * workgroup, 1 = one split over 8 waves; one-product, one bit per step: one form; two key
- * bits per step: 0 / 1 = two ciphertexts per workgroup, 2 = split; in a pbs_multibit = 3
- * context 0 / 1 are one bit per step and 2 / 3 / 4 those of two bits) of the
+ * workgroup, 1 = one split over 8 waves; one-product, one bit per step: 1, the one form; two key
+ * bits per step: 0 = two ciphertexts per workgroup, 2 = split; in a pbs_multibit = 3
+ * context 1 is one bit per step and 2 / 4 those of two bits) of the
  * full-round part and of the rest of tfhe_cbs_batch's split,
- * the PFKS i-slices of the same two parts, and the N=2048 key switch's i-slices;
+ * the PFKS i-slices of the same two parts (of their whole groups of 512 inputs), and the
+ * N=2048 key switch's i-slices;
  * -1 where a part does not exist.  A part of 16 or more rounds of resident
  * workgroups (8192 inputs on 256 CUs), or whose model shape takes over 250 ms per
  * launch, keeps the model shape without timing others.  Overwrites the context's AES state, RGSW and LUT
@@ -431,10 +432,12 @@ int tfhe_cbs_autotune(tfhe_cbs_ctx* ctx, uint32_t blocks, int* choices, void* st
  * tfhe_cbs_autotune's choices[0]; -1 returns that size to the size model), e.g. to
  * restore a stored autotune result without timing again.  No counterpart in the
  * reference (its shapes are compile-time).  TFHE_E_PARAM for a form the context's PBS
- * does not have.  Drops captured keystream graphs.  The FFT and key-batch forms of one
- * PBS give the same words, except the split form, whose two wave groups' partial sums
- * are added once (words differ by FP64 rounding); in a pbs_multibit = 3 context, choosing
- * one or two key bits per step changes them too (all decrypt within the PBS noise). */
+ * does not have; the numbers between those that the tuner reports stand for the same kernels
+ * (one bit 0 = 1, two bits 1 = 0, pbs_multibit = 3: 0 = 1 and 3 = 2).  Drops captured keystream
+ * graphs.  The forms of the exact PBS give the same words; the split form of two key bits per
+ * step adds its two wave groups' partial sums once (words differ by FP64 rounding), and in a
+ * pbs_multibit = 3 context choosing one or two key bits per step changes them too (all decrypt
+ * within the PBS noise). */
 int tfhe_cbs_set_pbs_form(tfhe_cbs_ctx* ctx, uint32_t inputs, int form);
 
 /* Kernel timing of the multi-value PBS (the reference prints per-block

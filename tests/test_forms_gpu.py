@@ -382,3 +382,23 @@ def test_one_product_forms_agree(gpu, okeys, form):
     assert err < 0.25
     assert apart(large[256], want) < 2 ** 40
     c.close()
+
+
+@pytest.mark.parametrize("params,forms", [({}, (0, 1)), ({"pbs_approx": 1}, (1,)),
+                                          ({"pbs_approx": 1, "pbs_multibit": 2}, (0, 2)),
+                                          ({"pbs_approx": 1, "pbs_multibit": 3}, (1, 2, 4))],
+                         ids=["exact", "one_bit", "two_bits", "auto"])
+def test_autotune_reports_each_kernel_by_one_number(gpu, okeys, params, forms):
+    """The tuner times each PBS kernel once: the choices of 1, 3 and 5 blocks (5: a full round and a
+    rest) name one of the context's kernels, never an alias, and the aliases stay accepted."""
+    import tfhe_amd
+    c = tfhe_amd.CbsContext(max_blocks=5, params=tfhe_amd.cbs_params(**params))
+    c.keygen(okeys.s, SEED)
+    for blocks in (1, 3, 5):
+        chosen = c.autotune(blocks)["pbs_form"]
+        assert all(f in forms for f in chosen[blocks < 5:]), (blocks, chosen)
+    for f in range(max(forms) + 1):
+        c.set_pbs_form(77, f)
+    with pytest.raises(tfhe_amd.TfheError):
+        c.set_pbs_form(77, 5 if params.get("pbs_multibit") == 3 else max(forms) + 1)
+    c.close()
