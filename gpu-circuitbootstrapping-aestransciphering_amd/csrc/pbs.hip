@@ -374,6 +374,7 @@ __global__ __launch_bounds__(256, 2) void k_pbs2(const uint32_t* __restrict__ lw
 template <int LIMBS, int MB, bool ANYM>
 struct PbsPair {
     using S = PbsStep<LIMBS, MB, ANYM>;
+    static_assert((LIMBS == 2) != (MB == 2), "the exact or the two-bit step: one limb and one bit run k_pbs2");
     static constexpr int NQ = ANYM ? 2 : 1;
     static constexpr int DEPTH = MB == 2 ? 2 : 4;  // key batches in flight
     cplx macc[2][2][LIMBS][2];       // [ciphertext][output][limb][q]
@@ -388,10 +389,8 @@ struct PbsPair {
             if constexpr (MB == 2) {
                 const int pt = b == 0 ? 0 : b == 1 ? 2 : 1;  // factors in the order (1,0), (1,1), (0,1)
                 k = key + ((size_t)(pt * PBS_ROWS + r) * 2 + o) * CB_M;
-            } else if constexpr (LIMBS == 2) {  // batch b: output b, limb o
+            } else {  // batch b: output b, limb o
                 k = key + ((size_t)(r * 2 + b) * 2 + o) * CB_M;
-            } else {
-                k = key + ((size_t)r * 2 + o) * CB_M;
             }
             kv[2 * o] = key_at(k, at);
             kv[2 * o + 1] = key_at(k + 512, at);
@@ -410,10 +409,7 @@ struct PbsPair {
                     for (int o = 0; o < 2; ++o) cmac_first(first, macc[c][o][0][q], y, kv[2 * o + q]);
                 } else {
 #pragma unroll
-                    for (int o = 0; o < 2; ++o) {
-                        if constexpr (LIMBS == 2) cmac_first(first, macc[c][b][o][q], x[c][q], kv[2 * o + q]);
-                        else cmac_first(first, macc[c][o][0][q], x[c][q], kv[2 * o + q]);
-                    }
+                    for (int o = 0; o < 2; ++o) cmac_first(first, macc[c][b][o][q], x[c][q], kv[2 * o + q]);
                 }
             }
     }
