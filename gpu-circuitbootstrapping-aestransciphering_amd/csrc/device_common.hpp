@@ -373,10 +373,4 @@ __host__ __device__ constexpr uint32_t digit_offset32() {
     return off;
 }
 
-template <int LOGB, int L>
-__device__ __forceinline__ int32_t digit32(uint32_t t_plus_off, int j) {
-    constexpr int IGN = 32 - L * LOGB;
-    return (int32_t)((t_plus_off >> (IGN + j * LOGB)) & ((1u << LOGB) - 1)) - (1 << (LOGB - 1));
-}
-
 }  // namespace tfhe

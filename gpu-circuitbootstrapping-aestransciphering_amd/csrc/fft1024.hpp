@@ -83,8 +83,6 @@ __device__ __forceinline__ cplx pw_const(int j) {
     return {c, j < 0 ? -s : s};
 }
 
-__device__ __forceinline__ int f256_a1(int k0, int b) { return k0 * 80 + (b >> 4) * 20 + (b & 15); }
-
 // The first transpose of the forward 256-point step (and the last of the inverse, its own
 // inverse): slot c of lane 16 q + d takes slot q of lane 16 c + d, a 4 x 4 transpose of
 // (slot, 16-lane row) done in registers by gfx950's row swaps: v_permlane32_swap exchanges
