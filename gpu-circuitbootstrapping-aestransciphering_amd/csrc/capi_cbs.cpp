@@ -212,6 +212,8 @@ struct tfhe_cbs_ctx {
     uint32_t tail_blocks = 0;
     hipEvent_t ev_gfork = nullptr, ev_gjoin = nullptr;
     DeviceTables1024 tables;
+    DeviceTables1024 exact_tables;  // of the exact PBS and its key (fft_tables.hpp); empty in one-product contexts
+    const FFT1024Tables& pbs_tables() const { return exact_tables.d_buf ? exact_tables.T : tables.T; }
     // AES state
     uint32_t max_blocks = 0;
     uint32_t* d_sbox_poly = nullptr;            // [N]
@@ -279,6 +281,7 @@ extern "C" int tfhe_cbs_ctx_destroy(tfhe_cbs_ctx* c) {
     if (c->cstream) (void)hipStreamDestroy(c->cstream);
     for (hipEvent_t e : c->tev) (void)hipEventDestroy(e);
     c->tables.release();
+    c->exact_tables.release();
     delete c;
     return TFHE_OK;
 }
@@ -344,6 +347,7 @@ extern "C" int tfhe_cbs_ctx_create(const tfhe_cbs_params* params, uint32_t max_b
     rc = rc ? rc : dmalloc((void**)&c->d_ctr, (size_t)max_blocks * 16);
     rc = rc ? rc : dmalloc((void**)&c->d_pub, (size_t)max_blocks * 16);
     rc = rc ? rc : c->tables.init();
+    if (pbs_limbs(p) == 2) rc = rc ? rc : c->exact_tables.init(true);
     if (!rc) {
         // S-box table packed for vertical packing: coefficient 8x + j = bit j of S(x), times 2^31
         std::vector<uint32_t> poly(kN, 0);
@@ -596,9 +600,9 @@ extern "C" int tfhe_cbs_set_keys(tfhe_cbs_ctx* c, const int32_t* rlwe_sk, const 
     if (!rc) rc = pack_kskl(c);
     if (!rc) {
         if (pbs_limbs(p) == 2)
-            launch_to_fourier2048(d_bsk, bsk2_rgsw(p) * 8 * 2, c->tables.T, c->d_bsk2f, nullptr);
+            launch_to_fourier2048(d_bsk, bsk2_rgsw(p) * 8 * 2, c->pbs_tables(), c->d_bsk2f, nullptr);
         else
-            launch_to_fourier2048_t64(d_bsk, bsk2_rgsw(p) * 8 * 2, c->tables.T, c->d_bsk2f, nullptr);
+            launch_to_fourier2048_t64(d_bsk, bsk2_rgsw(p) * 8 * 2, c->pbs_tables(), c->d_bsk2f, nullptr);
         rc = check_launch("set_keys fourier");
     }
     if (!rc) rc = hipcheck(hipDeviceSynchronize(), "set_keys sync");
@@ -638,9 +642,9 @@ extern "C" int tfhe_cbs_keygen(tfhe_cbs_ctx* c, const int32_t* lwe_sk, uint64_t 
                              p.bk_logB);
         }
         if (pbs_limbs(p) == 2)
-            launch_to_fourier2048(d_bsk, bsk2_rgsw(p) * 8 * 2, c->tables.T, c->d_bsk2f, nullptr);
+            launch_to_fourier2048(d_bsk, bsk2_rgsw(p) * 8 * 2, c->pbs_tables(), c->d_bsk2f, nullptr);
         else
-            launch_to_fourier2048_t64(d_bsk, bsk2_rgsw(p) * 8 * 2, c->tables.T, c->d_bsk2f, nullptr);
+            launch_to_fourier2048_t64(d_bsk, bsk2_rgsw(p) * 8 * 2, c->pbs_tables(), c->d_bsk2f, nullptr);
         if (htss(p)) {
             uint64_t* d_keys = nullptr;
             rc = dmalloc((void**)&d_keys, htss_key_words() * sizeof(uint64_t));
@@ -814,7 +818,7 @@ extern "C" int tfhe_cbs_pbs_batch(tfhe_cbs_ctx* c, const uint32_t* d_lwe, uint32
     hipEvent_t e1 = nullptr;
     rc = pbs_timing_begin(c, st, &e1);
     if (rc) return rc;
-    launch_pbs2(d_lwe, batch, c->p.n, bsk, pbs_limbs(c->p), mb, c->tables.T, d_out, st, form);
+    launch_pbs2(d_lwe, batch, c->p.n, bsk, pbs_limbs(c->p), mb, c->pbs_tables(), d_out, st, form);
     rc = check_launch("pbs2");
     return rc ? rc : pbs_timing_end(c, st, e1, batch);
 }
@@ -838,7 +842,7 @@ extern "C" int tfhe_cbs_bootstrap_many_lut(tfhe_cbs_ctx* c, const uint32_t* d_lw
     io.rlwe = d_out;
     io.bw = bitwidth;
     io.logB = c->p.bk_logB;
-    launch_pbs2(d_lwe, batch, c->p.n, bsk, pbs_limbs(c->p), mb, c->tables.T, nullptr, (hipStream_t)stream, form, io);
+    launch_pbs2(d_lwe, batch, c->p.n, bsk, pbs_limbs(c->p), mb, c->pbs_tables(), nullptr, (hipStream_t)stream, form, io);
     return check_launch("bootstrap_many_lut");
 }
 
@@ -926,7 +930,7 @@ static int cbs_batch_impl(tfhe_cbs_ctx* c, const CbsScratch& sc, const uint32_t*
         hipEvent_t e1 = nullptr;
         int rc = pbs_timing_begin(c, st, &e1);
         if (rc) return rc;
-        launch_pbs2(d_lwe, batch, c->p.n, c->d_bsk2f, 2, 1, c->tables.T, nullptr, st, tuned(c->tune_pbs, batch, -1),
+        launch_pbs2(d_lwe, batch, c->p.n, c->d_bsk2f, 2, 1, c->pbs_tables(), nullptr, st, tuned(c->tune_pbs, batch, -1),
                     htss_pbs_io(c, sc.lwe64));
         rc = check_launch("htss pbs");
         if (!rc) rc = pbs_timing_end(c, st, e1, batch);
@@ -1196,17 +1200,17 @@ extern "C" int tfhe_cbs_autotune(tfhe_cbs_ctx* c, uint32_t blocks, int* choices,
             rc = tune_one(st, e0, e1, cand, budget_ms,
                           [&](int f) {
                               if (f >= 2 && pbs_auto(c->p))
-                                  launch_pbs2(c->sc.state[0], batch, n, bsk2, limbs, 2, c->tables.T, c->sc.lwe64, st,
+                                  launch_pbs2(c->sc.state[0], batch, n, bsk2, limbs, 2, c->pbs_tables(), c->sc.lwe64, st,
                                               f - 2);
                               else
-                                  launch_pbs2(c->sc.state[0], batch, n, c->d_bsk2f, limbs, mb, c->tables.T,
+                                  launch_pbs2(c->sc.state[0], batch, n, c->d_bsk2f, limbs, mb, c->pbs_tables(),
                                               c->sc.lwe64, st, f, io);
                           },
                           form);
             if (!rc) c->tune_pbs[batch] = form;
         } else {
             // one form: its output still feeds the PFKS timing below
-            launch_pbs2(c->sc.state[0], batch, n, c->d_bsk2f, limbs, mb, c->tables.T, c->sc.lwe64, st, -1, io);
+            launch_pbs2(c->sc.state[0], batch, n, c->d_bsk2f, limbs, mb, c->pbs_tables(), c->sc.lwe64, st, -1, io);
             rc = check_launch("autotune pbs");
         }
         choices[part] = form;

@@ -12,6 +12,7 @@
 #include "device_common.hpp"
 #include "fft1024.hpp"
 #include "fft512_pair.hpp"
+#include "fft_tables.hpp"
 
 namespace tfhe {
 
@@ -108,43 +109,10 @@ struct DeviceTables {
 struct DeviceTables1024 {
     FFT1024Tables T{};
     cplx* d_buf = nullptr;
-    static constexpr int kCount = 1792 + 4096 + 160;
-    // host values of the tables, in device order
-    static std::vector<cplx> host_values() {
-        std::vector<cplx> h(kCount);
-        const double PI = 3.14159265358979323846264338327950288;
-        const int N = 2048;
-        auto put = [&](int idx, double ang) { h[idx] = {std::cos(ang), std::sin(ang)}; };
-        for (int k0 = 0; k0 < 4; ++k0)
-            for (int b = 0; b < 64; ++b)  // (w^4)^b * W256^(b k0)
-                put(k0 * 64 + b, PI * 4.0 * b / N - 2.0 * PI * (double)((b * k0) % 256) / 256.0);
-        for (int e = 0; e < 4; ++e)
-            for (int L = 0; L < 64; ++L) put(256 + e * 64 + L, -2.0 * PI * (double)(((L & 15) * e) % 64) / 64.0);
-        for (int p = 0; p < 4; ++p)
-            for (int L = 0; L < 64; ++L) put(512 + p * 64 + L, -2.0 * PI * (double)(((L & 3) * p) % 16) / 16.0);
-        for (int r = 0; r < 4; ++r)
-            for (int s = 0; s < 4; ++s)
-                for (int l = 0; l < 64; ++l) {
-                    const int k = (l >> 4) + 4 * ((l >> 2) & 3) + 16 * (l & 3) + 64 * s;
-                    put(768 + (r * 4 + s) * 64 + l, PI * r / N - 2.0 * PI * (double)((r * k) % 1024) / 1024.0);
-                }
-        for (int j = 0; j < 2 * N; ++j) put(1792 + j, PI * j / N);
-        for (int L = 0; L < 16; ++L) {
-            const int k = (L >> 2) + 4 * (L & 3);
-            auto pw = [&](int t, int p, int power) {  // (w^4 W256^(k + 16 p))^power, in units of pi / 512
-                put(1792 + 2 * N + t * 16 + L, PI * (double)(((1 - 4 * (k + 16 * p)) * power) % 1024) / 512.0);
-            };
-            pw(0, 0, 4);
-            pw(1, 0, 8);
-            for (int p = 0; p < 4; ++p) {
-                pw(2 + 2 * p, p, 1);
-                pw(3 + 2 * p, p, 2);
-            }
-        }
-        return h;
-    }
-    int init() {
-        const std::vector<cplx> h = host_values();
+    // rounded: fft_tables.hpp
+    int init(bool rounded = false) {
+        const std::vector<TableValue> h = fft1024_tables(rounded);
+        static_assert(sizeof(TableValue) == sizeof(cplx), "the tables' values are copied as they are");
         int rc = dmalloc((void**)&d_buf, h.size() * sizeof(cplx));
         if (rc) return rc;
         rc = hipcheck(hipMemcpy(d_buf, h.data(), h.size() * sizeof(cplx), hipMemcpyHostToDevice), "tables1024");
@@ -168,7 +136,7 @@ struct DeviceTables1024F {
     FFT1024TablesF T{};
     cplxf* d_buf = nullptr;
     int init() {
-        const std::vector<cplx> h = DeviceTables1024::host_values();
+        const std::vector<TableValue> h = fft1024_tables(false);
         std::vector<cplxf> f(h.size());
         for (size_t k = 0; k < h.size(); ++k) f[k] = {(float)h[k].re, (float)h[k].im};
         int rc = dmalloc((void**)&d_buf, f.size() * sizeof(cplxf));
