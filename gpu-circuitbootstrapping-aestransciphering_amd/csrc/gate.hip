@@ -128,11 +128,12 @@ __device__ __forceinline__ uint32_t gate_tv(uint32_t q1, uint32_t q2, uint32_t b
 
 // ===========================================================================
 // Persistent batched gate bootstrap: one wavefront owns one ciphertext for all n
-// blind-rotation steps, half-wave u its accumulator polynomial u.  Bound by FP64 issue (2,388
-// FP64 of 3,080 vector instructions per step, two waves per SIMD: 77% of the issue slots at
-// the clock the chip holds under FMA load).  With one radix-8 transform per wave at a time
+// blind-rotation steps, half-wave u its accumulator polynomial u.  Bound by FP64 issue and what two
+// waves per SIMD leave of its latency uncovered (2,388 FP64 of 3,080 vector instructions per step; at 4096
+// gates the vector unit is busy 71% of the time at the 2.0 GHz that the chip holds, the LDS 30%, a
+// sixth of that in bank conflicts; 256 registers, 11 spilled).  With one radix-8 transform per wave at a time
 // (two LDS round trips each, eight in a row) 1000 / 2048 / 4096 gates took 6.5 / 11.2 / 21.2 ms;
-// now 6.0 / 10.3 / 19.8 (the monic update's
+// now 6.0 / 10.3 / 20.2 (the monic update's
 // table values are loaded before the last keys, the inverse's 1 / M is in its factors).  Per step: the digit rows
 // of both polynomials by pairs (fft512_pair.hpp), the Fourier-domain MAC against the
 // streamed BSK row block, the two inverse transforms as one pair, exact rounding mod 2^32 and
@@ -778,8 +779,8 @@ void launch_to_fourier1024(const uint32_t* coef, size_t npoly, const FFTTables& 
     k_to_fourier1024<<<(unsigned)((npoly + 3) / 4), 256, 0, st>>>(coef, npoly, T, out);
 }
 
-// Largest batch of the 12-wave form: it takes 1.9-2.1 ms per round of one workgroup per CU,
-// the one-wave form 6.5 ms for up to 4 ciphertexts per CU, so up to three rounds.
+// Largest batch of the 12-wave form: three rounds of one workgroup per CU.  With the key switch a call
+// of 256 / 512 / 768 gates takes 2.1 / 3.9 / 5.7 ms; the one-wave form takes 6.4 up to 4 ciphertexts per CU.
 static uint32_t gate_split_max() { return 3 * device_cus(); }
 
 void launch_gate_blind_rotate(const uint32_t* ct1, const uint32_t* ct2, uint32_t batch, int n, int doubled,

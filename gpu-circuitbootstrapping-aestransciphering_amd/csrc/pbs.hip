@@ -806,7 +806,7 @@ __global__ __launch_bounds__(512, 1) void k_pbs2_split(const uint32_t* __restric
 // ===========================================================================
 int pbs_model_form(uint32_t batch, int limbs, int mb) {
     // Split over 8 waves (one limb, two bits: form 2; two limbs: form 1) up to one workgroup
-    // per CU, else two ciphertexts per workgroup (form 0): a second round of the split form, 3.3 ms for
+    // per CU (256 of them), else two ciphertexts per workgroup (form 0): a second round of the split form, 3.3 ms for
     // 256 inputs (exact 5.9), costs more than the paired form's one round of 512, 5.6 (10.8).
     if (mb == 2) return batch <= 256 ? 2 : 0;
     if (limbs == 2) return batch <= 256 ? 1 : 0;
